@@ -752,7 +752,8 @@ static int grow(gfl_ctx* c, hipStream_t st, void** buf, size_t* have, size_t nee
 static int grouped_workspace(gfl_ctx* c, hipStream_t st, int P, int M, int E, int H, int I, const char* who, Gws& w)
 {
     const size_t nch = (P + gfl::GP_PLAN_CHUNK - 1) / gfl::GP_PLAN_CHUNK;
-    const size_t n_int = 4 + (size_t)E + (E + 1) + 7 * (size_t)P + (size_t)M + (size_t)P + (size_t)E + nch * (E + 1);
+    const size_t n_it = (size_t)gfl::gemm_items(P, E, gfl::GP_MIN_MT);
+    const size_t n_int = 4 + 4 * n_it + 2 * (size_t)P + (size_t)E + (E + 1) + 8 * (size_t)P + (size_t)M + nch * (E + 1);
     const size_t b_int = align256(sizeof(int) * n_int);
     const size_t g_xt = align256(2 * 2 * (size_t)P * H), g_ygu = align256(2 * 2 * (size_t)P * I);
     const size_t g_xd = align256(2 * (size_t)P * I), g_yr = align256(2 * (size_t)P * H);
@@ -764,7 +765,9 @@ static int grouped_workspace(gfl_ctx* c, hipStream_t st, int P, int M, int E, in
     int* ip = reinterpret_cast<int*>(b);
     gfl::GPlan& gp = w.gp;
     gp.hdr = ip;
-    gp.cnt = gp.hdr + 4;
+    gp.item = reinterpret_cast<int4*>(gp.hdr + 4);
+    gp.tok_svh = reinterpret_cast<uint64_t*>(gp.item + n_it);
+    gp.cnt = gp.hdr + 4 + 4 * n_it + 2 * (size_t)P;
     gp.off = gp.cnt + E;
     gp.slot_pick = gp.off + E + 1;
     gp.slot_e = gp.slot_pick + P;
@@ -774,8 +777,7 @@ static int grouped_workspace(gfl_ctx* c, hipStream_t st, int P, int M, int E, in
     gp.tok_slot = gp.slot_job + P;
     gp.tok_w = reinterpret_cast<float*>(gp.tok_slot + P);
     gp.tok_npk = reinterpret_cast<int*>(gp.tok_w + P);
-    gp.eord = gp.tok_npk + M;
-    gp.ccnt = gp.eord + E;
+    gp.ccnt = gp.tok_npk + M;
     char* d = b + b_int;
     w.xt = reinterpret_cast<uint16_t*>(d);
     w.ygu16 = reinterpret_cast<uint16_t*>(d + g_xt);
@@ -894,7 +896,7 @@ int gfl_grouped_plan(gfl_ctx* c, const int64_t* sel, const void* w, int w_is_hal
     Gws ws;
     if (const int rc = grouped_workspace(c, st, P, M, E, 0, 0, "gfl_grouped_plan", ws)) return rc;
     const gfl::GPlan& gp = ws.gp;
-    gfl::launch_grouped_plan(sel, w, w_is_half ? 1 : 0, P, topk, E, gp, st);
+    gfl::launch_grouped_plan(nullptr, sel, w, w_is_half ? 1 : 0, P, topk, E, gfl::GP_MIN_MT, gp, st);
     GFL_HIP(hipGetLastError());
     GFL_HIP(hipMemcpyAsync(hdr, gp.hdr, 2 * sizeof(int), hipMemcpyDeviceToDevice, st));
     GFL_HIP(hipMemcpyAsync(off, gp.off, (E + 1) * sizeof(int), hipMemcpyDeviceToDevice, st));

@@ -103,7 +103,9 @@ int launch_dequant(const uint8_t* tr, int k, int n, int K, uint16_t* W, hipStrea
 // Grouped-rows plan of the prefill path (device arrays; P picks, E experts, M tokens).
 struct GPlan
 {
-    int* hdr;        // [0] slots S, [1] ids outside [-1, E)
+    int* hdr;        // [0] slots S, [1] ids outside [-1, E), [2] GEMM items
+    int4* item;      // [gemm_items] GEMM items {expert, first slot, slots, 0}: passes of up to mt slots of an expert,
+                     // whole passes first, then the remainders by descending size
     int* cnt;        // [E] slots of each expert
     int* off;        // [E + 1] slot offsets (experts ascending)
     int* slot_pick;  // [P] pick of each slot (picks ascending within an expert)
@@ -113,12 +115,17 @@ struct GPlan
     int* slot_job;   // [P] reference job number (combine order), set at the slots of job-opening picks
     int* tok_slot;   // [M][topk] slots of each token in combine order
     float* tok_w;    // [M][topk] their routing weights (fp32)
+    uint64_t* tok_svh;   // [M][topk] their experts' svh_down addresses
     int* tok_npk;    // [M] valid picks of each token
-    int* eord;       // [E] experts in GEMM dispatch order: most slots first, then ascending id
     int* ccnt;       // [chunks][E + 1] picks of each expert per chunk of GP_PLAN_CHUNK picks, other ids at [E]
 };
 
 constexpr int GP_PLAN_CHUNK = 1024;   // picks per workgroup of the grouped plan
+
+// Most GEMM items that P picks over E experts can make with passes of mt slots: P / mt whole passes, and a remainder
+// of each expert that has picks.
+constexpr int gemm_items(int P, int E, int mt) { return P / mt + (P < E ? P : E); }
+constexpr int GP_MIN_MT = 16;   // fewest slots per pass of any GEMM on the grouped plan
 
 // Prefill-sized layer forward with MFMA grouped GEMMs (k_prefill.hip): xt [2][cap][H] fp16, ygu [2][cap][I] fp16,
 // xd [cap][I] fp16, yraw [cap][H] fp16 workspace, cap >= P. The GEMM outputs ygu and yraw are stored rounded to fp16,
@@ -138,8 +145,9 @@ int launch_exact_chains(const uint64_t* ptrs, const int64_t* sel, const void* w,
                         uint16_t* ygu, float* xd, uint16_t* yraw, const float* silu_tab, float act_limit, float* out,
                         hipStream_t st);
 // The grouped plan alone (first three launches of launch_grouped): slots, offsets, job order per token.
-void launch_grouped_plan(const int64_t* sel, const void* w, int w_half, int P, int topk, int E, const GPlan& g,
-                         hipStream_t st);
+// ptrs may be NULL (tok_svh is then 0).
+void launch_grouped_plan(const uint64_t* ptrs, const int64_t* sel, const void* w, int w_half, int P, int topk, int E,
+                         int mt, const GPlan& g, hipStream_t st);
 
 int launch_split(const int64_t* sel, const uint16_t* w, const uint16_t* z, int n, int bsz, int topk, int H, int E,
                  int first, const int32_t* slotof, const float* score, const float* pol, int64_t* ctrl, uint16_t* hx,

@@ -13,6 +13,7 @@
 // for tile row 2q + {0, 1, 8, 9}[jj]; the inputs are stored with the same row permutation ([tk][q][jj] per tile row),
 // so each decoded tile feeds the MFMA directly, with no transpose. gfx950's v_mfma_f32_16x16x32_f16 takes two such
 // slices (tile rows r and r + 1) per lane as its 8 k-values.
+#include <algorithm>
 #include <type_traits>
 
 #include "gfl_device.hpp"
@@ -33,8 +34,9 @@ constexpr int GP_ORDER_THREADS = 256;
 // [0, E) are skipped (ids other than -1 are counted in hdr[1]). The combine order of a token's picks is the
 // reference's job order: moe_forward (ft_core.h:1343-1349) scans picks token-major and opens a job for an expert at
 // its first pick and after every 8 of its picks, so pick p (the c-th of its expert) lands in the job opened by that
-// expert's pick number c - c % 8, and jobs are numbered in the order their opening picks appear. The plan takes three
-// launches over chunks of GP_PLAN_CHUNK picks: ranks within each chunk, then placement (every chunk sums the counts
+// expert's pick number c - c % 8, and jobs are numbered in the order their opening picks appear. A call of one chunk
+// takes one launch (gp_plan_kernel: 6.9 us against 31 us of the three at 184 picks), a longer one three launches over
+// chunks of GP_PLAN_CHUNK picks: ranks within each chunk, then placement (every chunk sums the counts
 // of the chunks before it), then each token's picks in job order.
 
 // Bit mask of the lanes below this one.
@@ -100,17 +102,55 @@ __device__ __forceinline__ int gp_wave_scan(int v, int lane)
     return v;
 }
 
+// The GEMM's items: every expert's slots in passes of mt, a workgroup per pass (and column block), so that an expert
+// with many slots runs its passes side by side. Whole passes first, then the remainders by descending size: the longest
+// workgroups go first and the short ones fill the end of the launch. The remainders are placed by a counting sort over
+// their sizes (mt <= 127; ties in any order, the items are independent). Comparing every expert with every other
+// instead took about 10 us of the plan at E = 288. Whole workgroup of GP_PLAN_THREADS, thread t = expert t: tot slots
+// from slot off; s_hist and s_full are LDS scratch; ends with a barrier.
+__device__ __forceinline__ void gp_items(int t, int E, int mt, int tot, int off, const GPlan& g, int* s_hist,
+                                         int* s_full)
+{
+    const int lane = t & 63, wv = t >> 6;
+    const int full = t < E ? tot / mt : 0, rem = t < E ? tot - full * mt : 0;
+    if (t < 128) s_hist[t] = 0;
+    const int finc = gp_wave_scan(full, lane);
+    if (lane == 63) s_full[wv] = finc;
+    __syncthreads();
+    int at = 0;   // place among the remainders of the same size
+    if (rem > 0) at = atomicAdd(&s_hist[rem], 1);
+    int fpre = 0, nfull = 0;
+    for (int v = 0; v < GP_PLAN_WAVES; ++v)
+    {
+        fpre += v < wv ? s_full[v] : 0;
+        nfull += s_full[v];
+    }
+    __syncthreads();
+    if (wv == 0)
+    {
+        const int v0 = s_hist[127 - 2 * lane], v1 = s_hist[126 - 2 * lane];   // sizes descending over the lanes
+        const int inc = gp_wave_scan(v0 + v1, lane);
+        s_hist[127 - 2 * lane] = inc - v0 - v1;
+        s_hist[126 - 2 * lane] = inc - v1;
+        if (lane == 63) g.hdr[2] = nfull + inc;
+    }
+    __syncthreads();
+    const int f0 = fpre + finc - full;
+    for (int k = 0; k < full; ++k) g.item[f0 + k] = make_int4(t, off + k * mt, mt, 0);
+    if (rem > 0) g.item[nfull + s_hist[rem] + at] = make_int4(t, off + full * mt, rem, 0);
+}
+
 // Pass 2, one workgroup per chunk: expert e's picks in earlier chunks (base_e) and in all chunks (its slot count),
 // slot offsets by a scan of the counts, and the jobs opened before the chunk, sum over e of ceil(base_e / 8) (the
 // expert's ranks 0, 8, 16, ... below base_e); a pick's global rank is base_e plus its rank in the chunk, and a pick
 // of rank r opens a job when r % 8 == 0, numbered after the chunk's earlier openers. Workgroup 0 also writes the
-// counts, offsets, header and the GEMM's expert order.
+// counts, offsets, header and the GEMM's items (passes of up to mt slots of an expert).
 __global__ __launch_bounds__(GP_PLAN_THREADS) void gp_place_kernel(const int64_t* __restrict__ sel, int P, int E,
-                                                                   GPlan g)
+                                                                   int mt, GPlan g)
 {
     __shared__ int s_base[MAX_EXPERTS];
     __shared__ int s_off[MAX_EXPERTS];
-    __shared__ __align__(16) int s_nsl[MAX_EXPERTS];
+    __shared__ int s_hist[128];
     __shared__ int s_wtot[GP_PLAN_WAVES], s_wjob[GP_PLAN_WAVES], s_wop[GP_PLAN_WAVES];
     __shared__ int s_bad;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
@@ -166,20 +206,9 @@ __global__ __launch_bounds__(GP_PLAN_THREADS) void gp_place_kernel(const int64_t
     __syncthreads();
     if (c == 0)
     {
-        // experts by descending slot count, ties by ascending id: a GEMM workgroup's time grows with its expert's
-        // slots (passes, and the blocks of the last pass), so the longest workgroups go first and the short ones
-        // fill the end of the launch
         if (t == 0) g.hdr[1] = s_bad;
-        s_nsl[t] = t < E ? tot : -1;
-        __syncthreads();
-        int rk = 0;
-        for (int k = 0; k < E; k += 4)   // 16-byte broadcast reads; entries past E are -1
-        {
-            const int4 pk = *reinterpret_cast<const int4*>(&s_nsl[k]);
-            rk += (pk.x > tot || (pk.x == tot && k < t)) + (pk.y > tot || (pk.y == tot && k + 1 < t)) +
-                  (pk.z > tot || (pk.z == tot && k + 2 < t)) + (pk.w > tot || (pk.w == tot && k + 3 < t));
-        }
-        if (t < E) g.eord[rk] = t;
+        gp_items(t, E, mt, tot, off_e, g, s_hist, s_wop);
+        __syncthreads();   // s_wop is used again below
     }
     const int r = ok ? s_base[e] + rc : 0;
     const bool opener = ok && (r & 7) == 0;
@@ -205,7 +234,8 @@ __global__ __launch_bounds__(GP_PLAN_THREADS) void gp_place_kernel(const int64_t
 
 // Pass 3, one thread per token: its picks in (job, pick) order with their fp32 weights. A pick of global rank c
 // reads its job number from the slot of its job's opening pick, c % 8 slots before its own.
-__global__ __launch_bounds__(GP_ORDER_THREADS) void gp_order_kernel(const void* w, int w_half, int M, int topk, GPlan g)
+__global__ __launch_bounds__(GP_ORDER_THREADS) void gp_order_kernel(const uint64_t* __restrict__ ptrs,
+                                                                    const void* w, int w_half, int M, int topk, GPlan g)
 {
     const int tk = blockIdx.x * GP_ORDER_THREADS + threadIdx.x;
     if (tk >= M) return;
@@ -232,19 +262,125 @@ __global__ __launch_bounds__(GP_ORDER_THREADS) void gp_order_kernel(const void* 
             r += ps[k2] >= 0 && (jb[k2] < jb[k] || (jb[k2] == jb[k] && k2 < k));
         const int p = tk * topk + k;
         g.tok_slot[tk * topk + r] = ps[k];
+        g.tok_svh[tk * topk + r] = ptrs ? ptrs[(size_t)g.slot_e[ps[k]] * 9 + 8] : 0;
         g.tok_w[tk * topk + r] = w_half ? h2f_bits(reinterpret_cast<const uint16_t*>(w)[p])
                                         : reinterpret_cast<const float*>(w)[p];
     }
 }
 
+// The three passes in one launch for a call of one chunk (P <= GP_PLAN_CHUNK): one workgroup, a thread per pick (and per
+// expert). Ranks as gp_rank_kernel, placement as gp_place_kernel with nothing before the chunk, and each pick's place in
+// its token's (job, pick) order by counting the token's picks before it.
+__global__ __launch_bounds__(GP_PLAN_THREADS) void gp_plan_kernel(const uint64_t* __restrict__ ptrs,
+                                                                  const int64_t* __restrict__ sel, const void* w,
+                                                                  int w_half, int P, int topk, int E, int mt, GPlan g)
+{
+    __shared__ unsigned char s_wcnt[GP_PLAN_WAVES][MAX_EXPERTS];   // group sizes (<= 64) of each wave
+    __shared__ int s_off[MAX_EXPERTS];
+    __shared__ int s_job[GP_PLAN_THREADS];    // job number of the slot, at the slots of job-opening picks
+    __shared__ int s_pjob[GP_PLAN_THREADS];   // each pick's job, -1 if skipped
+    __shared__ int s_hist[128];
+    __shared__ int s_wtot[GP_PLAN_WAVES], s_wop[GP_PLAN_WAVES], s_full[GP_PLAN_WAVES];
+    __shared__ int s_bad;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int64_t e64 = t < P ? sel[t] : -1;
+    float wt = 0.f;
+    if (t < P) wt = w_half ? h2f_bits(reinterpret_cast<const uint16_t*>(w)[t]) : reinterpret_cast<const float*>(w)[t];
+    if (t == 0) s_bad = 0;
+    for (int i = t; i < GP_PLAN_WAVES * MAX_EXPERTS / 4; i += GP_PLAN_THREADS)
+        reinterpret_cast<int*>(&s_wcnt[0][0])[i] = 0;
+    const bool ok = e64 >= 0 && e64 < E;
+    const int e = ok ? (int)e64 : 0;
+    const uint64_t svh = ok && ptrs ? ptrs[(size_t)e * 9 + 8] : 0;
+    uint64_t eq = __ballot(ok);
+#pragma unroll
+    for (int b = 0; b < 10; ++b)
+    {
+        const bool bit = ok && ((e >> b) & 1);
+        const uint64_t m = __ballot(bit);
+        eq &= bit ? m : ~m;
+    }
+    const int cin = __popcll(eq & gp_lanes_below(lane));
+    __syncthreads();
+    if (ok && cin == 0) s_wcnt[wv][e] = (unsigned char)__popcll(eq);
+    else if (!ok && e64 != -1) atomicAdd(&s_bad, 1);
+    __syncthreads();
+    int r = cin, tot = 0;
+#pragma unroll
+    for (int v = 0; v < GP_PLAN_WAVES; ++v)
+    {
+        r += v < wv ? s_wcnt[v][e] : 0;
+        tot += s_wcnt[v][t];
+    }
+    if (t >= E) tot = 0;
+    const int inc = gp_wave_scan(tot, lane);
+    const bool opener = ok && (r & 7) == 0;
+    const uint64_t om = __ballot(opener);
+    if (lane == 63) s_wtot[wv] = inc;
+    if (lane == 0) s_wop[wv] = __popcll(om);
+    __syncthreads();
+    int off_e = inc - tot, job = __popcll(om & gp_lanes_below(lane));
+    for (int v = 0; v < wv; ++v)
+    {
+        off_e += s_wtot[v];
+        job += s_wop[v];
+    }
+    s_off[t] = off_e;
+    if (t < E)
+    {
+        g.cnt[t] = tot;
+        g.off[t] = off_e;
+        if (t == E - 1)
+        {
+            g.off[E] = off_e + tot;
+            g.hdr[0] = off_e + tot;
+        }
+    }
+    if (t == 0) g.hdr[1] = s_bad;
+    gp_items(t, E, mt, tot, off_e, g, s_hist, s_full);   // its first barrier also orders s_off
+    const int s = ok ? s_off[e] + r : -1;
+    if (opener) s_job[s] = job;
+    __syncthreads();
+    const int jb = ok ? s_job[s - (r & 7)] : -1;
+    s_pjob[t] = jb;
+    if (t < P)
+    {
+        g.pick_slot[t] = s;
+        if (ok)
+        {
+            g.slot_pick[s] = t;
+            g.slot_e[s] = e;
+        }
+    }
+    __syncthreads();
+    if (t >= P) return;
+    const int tk = t / topk, k = t - tk * topk;
+    int rank = 0, npk = 0;
+    for (int k2 = 0; k2 < topk; ++k2)
+    {
+        const int j2 = s_pjob[tk * topk + k2];
+        npk += j2 >= 0;
+        rank += j2 >= 0 && (j2 < jb || (j2 == jb && k2 < k));
+    }
+    if (ok)
+    {
+        g.tok_slot[tk * topk + rank] = s;
+        g.tok_w[tk * topk + rank] = wt;
+        g.tok_svh[tk * topk + rank] = svh;
+    }
+    if (k == 0) g.tok_npk[tk] = npk;
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // transforms: one wave per slot, or per (token, group of blocks); each 16-lane row of the wave takes one 128-block,
-// 8 elements per lane (16-byte loads), 4 blocks per round; exact rounding points
+// 8 elements per lane (16-byte loads), 4 blocks per round; exact rounding points. Small calls are bound by the latency of
+// their dependent loads and give a slot to more waves (184 picks: input transform 11.4 -> 6.4 us, SwiGLU 9.9 -> 6.0 us)
 // ---------------------------------------------------------------------------------------------------------------
 
 constexpr int GP_TW = 4;   // waves per transform workgroup
 constexpr int GP_TU = 2;   // rounds of 4 blocks per chunk of the input transform (two chunks' loads in flight)
 constexpr int GP_TA = 3;   // rounds of 4 blocks per SwiGLU-transform wave (one wave covers I = 1536)
+constexpr int GP_SMALL = 1024;   // picks up to which a SwiGLU-transform wave takes one round
 
 // Elements 8li..8li+7 of 128-block b (one lane of a 16-lane row), rounded to fp16, into the accumulator-chain input
 // layout: fp32, position tk * 16 + 4j + q holds row 2q + {0, 1, 8, 9}[j] of tile row tk (the rows chain j of every
@@ -259,20 +395,24 @@ __device__ __forceinline__ void xg_store_row(float* dst, int b, int li, const fl
     *reinterpret_cast<float4*>(d + 4) = float4{ r[1], r[3], r[5], r[7] };
 }
 
-// prep_block (ft_core.h:97-102) of the gate and up inputs of slot s (one wave per slot). XL: fp32 in the
+// prep_block (ft_core.h:97-102) of the gate and up inputs of slot s, `parts` waves per slot (prep_parts). XL: fp32 in the
 // accumulator-chain layout (xg_store_row), else fp16 in the MFMA layout (gp_store_row).
 template <bool XL>
 __global__ __launch_bounds__(GP_TW * 64) void gp_prep_kernel(const uint64_t* __restrict__ ptrs,
                                                              const uint16_t* __restrict__ x, int H, int topk, int cap,
-                                                             GPlan g, void* __restrict__ xt_out)
+                                                             int parts, GPlan g, void* __restrict__ xt_out)
 {
     uint16_t* xt = static_cast<uint16_t*>(xt_out);
     float* xtf = static_cast<float*>(xt_out);
     const int lane = threadIdx.x & 63, rl = lane >> 4, li = lane & 15;
-    const int s = blockIdx.x * GP_TW + (threadIdx.x >> 6);
+    const int w = blockIdx.x * GP_TW + (threadIdx.x >> 6), s = w / parts;
+    const int e = g.slot_e[s], pick = g.slot_pick[s];   // read beside the slot count: past it stale entries, not used
     if (s >= g.hdr[0]) return;
-    const int nblk = H / 128;
-    const int e = g.slot_e[s], tok = g.slot_pick[s] / topk;
+    constexpr int CH = 4 * GP_TU;   // blocks per chunk
+    const int nall = H / 128, span = (nall + parts * CH - 1) / (parts * CH) * CH;
+    const int b0 = (w - s * parts) * span, nblk = min(nall, b0 + span);   // this wave's blocks [b0, nblk)
+    if (b0 >= nblk) return;
+    const int tok = pick / topk;
     const gptr<uint16_t> su0 = gaddr<uint16_t>(ptrs[(size_t)e * 9 + 3]);
     const gptr<uint16_t> su1 = gaddr<uint16_t>(ptrs[(size_t)e * 9 + 5]);
     const uint16_t* xr = x + (size_t)tok * H;
@@ -280,7 +420,6 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_prep_kernel(const uint64_t* __r
     uint16_t* d1 = xt + ((size_t)cap + s) * H;
     float* f0 = xtf + (size_t)s * H;
     float* f1 = xtf + ((size_t)cap + s) * H;
-    constexpr int CH = 4 * GP_TU;   // blocks per chunk
     uint4 xv[2][GP_TU], g0[2][GP_TU], g1[2][GP_TU];
     auto load = [&](int buf, int c0) {
 #pragma unroll
@@ -322,8 +461,8 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_prep_kernel(const uint64_t* __r
         }
     };
     // two chunk buffers: the next chunk's loads are in flight while the current one is transformed
-    load(0, 0);
-    for (int c0 = 0; c0 < nblk; c0 += 2 * CH)
+    load(0, b0);
+    for (int c0 = b0; c0 < nblk; c0 += 2 * CH)
     {
         if (c0 + CH < nblk) load(1, c0 + CH);
         work(0, c0);
@@ -332,20 +471,20 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_prep_kernel(const uint64_t* __r
     }
 }
 
-// fwd_phase phase 1 (ft_core.h:974-991), one wave per (slot, 4 * GP_TA blocks of I): per 128-block, out_block of
+// fwd_phase phase 1 (ft_core.h:974-991), one wave per (slot, 4 * TA blocks of I): per 128-block, out_block of
 // gate and up, r16(act_mul), down prep_block, stored in the GEMM input layout
-template <bool XL>
+template <bool XL, int TA>
 __global__ __launch_bounds__(GP_TW * 64) void gp_act_kernel(const uint64_t* __restrict__ ptrs, int I, int cap, GPlan g,
                                                             const uint16_t* __restrict__ ygu, const float* silu_tab,
                                                             float act_limit, void* __restrict__ xd_out)
 {
     uint16_t* xd = static_cast<uint16_t*>(xd_out);
     const int lane = threadIdx.x & 63, rl = lane >> 4, li = lane & 15;
-    const int nbi = I / 128, nch = (nbi + 4 * GP_TA - 1) / (4 * GP_TA);
+    const int nbi = I / 128, nch = (nbi + 4 * TA - 1) / (4 * TA);
     const int item = blockIdx.x * GP_TW + (threadIdx.x >> 6);
-    const int s = item / nch, c0 = (item % nch) * 4 * GP_TA;
+    const int s = item / nch, c0 = (item % nch) * 4 * TA;
+    const int e = g.slot_e[s];   // read beside the slot count: past it a stale entry, not used
     if (s >= g.hdr[0]) return;
-    const int e = g.slot_e[s];
     const gptr<uint16_t> svh_g = gaddr<uint16_t>(ptrs[(size_t)e * 9 + 4]);
     const gptr<uint16_t> svh_u = gaddr<uint16_t>(ptrs[(size_t)e * 9 + 6]);
     const gptr<uint16_t> suh_d = gaddr<uint16_t>(ptrs[(size_t)e * 9 + 7]);
@@ -353,14 +492,14 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_act_kernel(const uint64_t* __re
     const uint16_t* yu = ygu + ((size_t)cap + s) * I;
     uint16_t* dst = xd + (size_t)s * I;
     float* dstf = static_cast<float*>(xd_out) + (size_t)s * I;
-    // GP_TA rounds of 4 blocks in three phases kept apart by scheduling barriers (left to itself the compiler sinks
+    // TA rounds of 4 blocks in three phases kept apart by scheduling barriers (left to itself the compiler sinks
     // each round's loads next to their use): all loads; the output transforms and every silu lookup; the
     // activation, input transform and stores
     {
-        float gv[GP_TA][8], uv[GP_TA][8], ev[GP_TA][8];
-        uint4 gh[GP_TA], uh[GP_TA], sg[GP_TA], su[GP_TA], sd[GP_TA];
+        float gv[TA][8], uv[TA][8], ev[TA][8];
+        uint4 gh[TA], uh[TA], sg[TA], su[TA], sd[TA];
 #pragma unroll
-        for (int k = 0; k < GP_TA; ++k)
+        for (int k = 0; k < TA; ++k)
         {
             const int o = min(c0 + 4 * k + rl, nbi - 1) * 128 + li * 8;
             gh[k] = *reinterpret_cast<const uint4*>(yg + o);
@@ -371,18 +510,18 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_act_kernel(const uint64_t* __re
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int k = 0; k < GP_TA; ++k)
+        for (int k = 0; k < TA; ++k)
         {
             out_block_row_h(gv[k], gh[k], sg[k]);
             out_block_row_h(uv[k], uh[k], su[k]);
         }
 #pragma unroll
-        for (int k = 0; k < GP_TA; ++k)
+        for (int k = 0; k < TA; ++k)
 #pragma unroll
             for (int j = 0; j < 8; ++j) ev[k][j] = silu_tab[f2h_bits(gv[k][j]) & 0xFFFFu];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int k = 0; k < GP_TA; ++k)
+        for (int k = 0; k < TA; ++k)
         {
             const int b = c0 + 4 * k + rl;
             float av[8];
@@ -405,12 +544,11 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_act_kernel(const uint64_t* __re
 
 // out_block (ft_core.h:1016) of every expert output block and the weighted sum in job order (ft_core.h:1020-1033),
 // one wave per (token, group of 4 blocks): each 16-lane row takes one block; lane k < npk holds the token's k-th pick
-// (slot, weight, output scales), read back per pick with readlane; four picks' loads are issued before their four
-// terms are added in order. Rows of tokens without a valid pick become 0.
-constexpr int GP_CK = 4;   // picks whose loads a combine wave keeps in flight
+// (slot, weight, output scales), read back per pick with readlane; eight picks' loads are issued before their eight
+// terms are added in order (against four: M = 2048 47.2 -> 46.1 us). Rows of tokens without a valid pick become 0.
+constexpr int GP_CK = 8;   // picks whose loads a combine wave keeps in flight (all of a top-8 token's)
 
-__global__ __launch_bounds__(GP_TW * 64) void gp_comb_kernel(const uint64_t* __restrict__ ptrs, int H, int M, int topk,
-                                                             GPlan g, const uint16_t* __restrict__ yraw,
+__global__ __launch_bounds__(GP_TW * 64) void gp_comb_kernel(int H, int M, int topk, GPlan g, const uint16_t* __restrict__ yraw,
                                                              float* __restrict__ out)
 {
     const int lane = threadIdx.x & 63, rl = lane >> 4, li = lane & 15;
@@ -419,15 +557,11 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_comb_kernel(const uint64_t* __r
     const int tok = item / ngr, b = (item % ngr) * 4 + rl;
     if (tok >= M) return;
     const int npk = g.tok_npk[tok];
-    int my_s = 0;
-    float my_w = 0.f;
-    uint64_t my_p = 0;
-    if (lane < npk)
-    {
-        my_s = g.tok_slot[tok * topk + lane];
-        my_w = g.tok_w[tok * topk + lane];
-        my_p = ptrs[(size_t)g.slot_e[my_s] * 9 + 8];
-    }
+    // entries past the token's picks hold stale values, which are not used
+    const int ml = tok * topk + min(lane, topk - 1);
+    const int my_s = g.tok_slot[ml];
+    const float my_w = g.tok_w[ml];
+    const uint64_t my_p = g.tok_svh[ml];
     const int o = min(b, nbh - 1) * 128 + li * 8;
     float acc[8];
 #pragma unroll
@@ -488,15 +622,15 @@ __device__ __forceinline__ void gp_wait_vmcnt()
 
 // Workgroup barrier without __syncthreads' release fence: that fence waits for vmcnt(0), i.e. for every LDS-direct
 // load still in flight, which would drain the prefetch ring at every group. Each wave has already waited for its own
-// loads of the group it is about to read; the barrier only has to order those waits (and the previous group's LDS
-// reads) across the waves. The "memory" clobber keeps the compiler from moving LDS accesses across it.
-__device__ __forceinline__ void gp_barrier() { asm volatile("s_barrier" ::: "memory"); }
+// loads of the group it is about to read; the barrier only has to order those waits and the previous group's LDS
+// reads (waited for here, nothing else is outstanding on that counter) across the waves. The "memory" clobber keeps the compiler from moving LDS accesses across it.
+__device__ __forceinline__ void gp_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 struct GemmArgs
 {
     const uint64_t* ptrs;
     int mat_base, nmat;        // first matrix of the launch (0 gate, 1 up, 2 down) and how many
-    int kdim, ndim, cap, E;
+    int kdim, ndim, cap, nit;  // nit: items the grid covers
     GPlan g;
     const uint16_t* xin;       // [mats][cap][kdim] fp16, GEMM input layout
     uint16_t* yout;            // [mats][cap][ndim] fp16: out_block's leading r16 (ft_core.h:109) applied here
@@ -523,13 +657,12 @@ __global__ __launch_bounds__(GP_NW * 64) void gp_gemm_kernel(GemmArgs a)
     // are fetched into one L2
     const int nch = a.ndim / GP_WCOLS, per = nch * a.nmat;
     const int xcd = blockIdx.x % 8, j = blockIdx.x / 8;
-    const int ei = (j / per) * 8 + xcd, rr0 = j % per;
-    if (ei >= a.E) return;
-    const int e = a.g.eord[ei];   // experts with the most slots first
+    const int it = (j / per) * 8 + xcd, rr0 = j % per;
+    if (it >= a.nit || it >= a.g.hdr[2]) return;
+    const int4 item = a.g.item[it];   // a pass of up to GP_MT slots of an expert
+    const int e = item.x, c0 = item.y, T = item.z;
     const int nc = rr0 % nch;
     const int mat = a.mat_base + rr0 / nch;
-    const int s_begin = a.g.off[e], s_end = a.g.off[e + 1];
-    if (s_begin >= s_end) return;
     const int TN = a.ndim / 16, TK = a.kdim / 16, ngroups = TK / 8;
     const int t0 = (nc * GP_NW + wave) * GP_CPW;                     // this wave's first tile column
     uint8_t* ring = gp_lds + wave * NG * GB;                          // [NG][8 tile rows][GP_CPW columns][TB]
@@ -557,112 +690,107 @@ __global__ __launch_bounds__(GP_NW * 64) void gp_gemm_kernel(GemmArgs a)
     uint16_t* yout = a.yout + (size_t)(mat - a.mat_base) * a.cap * a.ndim;
     const int q = lane >> 4, i16 = lane & 15;
 
-    for (int c0 = s_begin; c0 < s_end; c0 += GP_MT)
-    {
-        const int T = min(GP_MT, s_end - c0);
-        // byte offsets of the input rows this wave loads, the same in every lane (slots past the pass read the pass's
-        // last slot): the scalar offset of its LDS-direct loads, whose vector offset is the lane's 4 bytes
-        int xrow[GP_XPW];
+    // byte offsets of the input rows this wave loads, the same in every lane (slots past the pass read the pass's
+    // last slot): the scalar offset of its LDS-direct loads, whose vector offset is the lane's 4 bytes
+    int xrow[GP_XPW];
 #pragma unroll
-        for (int j = 0; j < GP_XPW; ++j) xrow[j] = (c0 + min(wave * GP_XPW + j, T - 1)) * a.kdim * 2;
-        const int xl = lane * 4;
-        auto issue = [&](int g) {
-            uint8_t* dst = ring + (g % NG) * GB;
+    for (int j = 0; j < GP_XPW; ++j) xrow[j] = (c0 + min(wave * GP_XPW + j, T - 1)) * a.kdim * 2;
+    const int xl = lane * 4;
+    auto issue = [&](int g) {
+        uint8_t* dst = ring + (g % NG) * GB;
 #pragma unroll
-            for (int i = 0; i < NLD; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (gp_lds_void*)(dst + i * 256), 4, voff[i], g * 8 * gs, 0,
-                                                         0);
-            uint16_t* xd = xring + (size_t)(g % NG) * GP_MT * GP_XS;
+        for (int i = 0; i < NLD; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (gp_lds_void*)(dst + i * 256), 4, voff[i], g * 8 * gs, 0,
+                                                     0);
+        uint16_t* xd = xring + (size_t)(g % NG) * GP_MT * GP_XS;
 #pragma unroll
-            for (int j = 0; j < GP_XPW; ++j)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (gp_lds_void*)(xd + (wave * GP_XPW + j) * GP_XS), 4, xl,
-                                                         xrow[j] + g * 256, 0, 0);
-        };
-        // the pass with its NMB = ceil(T / 16) row blocks of 16 slots: MFMAs and input fragments of empty blocks
-        // are not issued
-        auto pass = [&](auto nmb_c) {
-            constexpr int NMB = decltype(nmb_c)::value;
-            float4v acc[GP_CPW][NMB];
+        for (int j = 0; j < GP_XPW; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (gp_lds_void*)(xd + (wave * GP_XPW + j) * GP_XS), 4, xl,
+                                                     xrow[j] + g * 256, 0, 0);
+    };
+    // the pass with its NMB = ceil(T / 16) row blocks of 16 slots: MFMAs and input fragments of empty blocks
+    // are not issued
+    auto pass = [&](auto nmb_c) {
+        constexpr int NMB = decltype(nmb_c)::value;
+        float4v acc[GP_CPW][NMB];
 #pragma unroll
-            for (int c = 0; c < GP_CPW; ++c)
+        for (int c = 0; c < GP_CPW; ++c)
 #pragma unroll
-                for (int mb = 0; mb < NMB; ++mb) acc[c][mb] = float4v{ 0.f, 0.f, 0.f, 0.f };
-            __syncthreads();   // previous pass done with the rings
+            for (int mb = 0; mb < NMB; ++mb) acc[c][mb] = float4v{ 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
-            for (int g = 0; g < NG - 1; ++g)
-                if (g < ngroups) issue(g);
-            for (int g = 0; g < ngroups; ++g)
+        for (int g = 0; g < NG - 1; ++g)
+            if (g < ngroups) issue(g);
+        for (int g = 0; g < ngroups; ++g)
+        {
+            if (g + NG - 2 < ngroups) gp_wait_vmcnt<(NG - 2) * NV>();   // this wave's loads of group g landed
+            else gp_wait_vmcnt<0>();
+            gp_barrier();   // every wave's loads of group g landed; every wave is done with group g - 1
+            if (g + NG - 1 < ngroups) issue(g + NG - 1);   // into the slots of group g - 1
+            const uint8_t* sl = ring + (g % NG) * GB;
+            const uint16_t* xs = xring + (size_t)(g % NG) * GP_MT * GP_XS;
+#pragma unroll
+            for (int rp = 0; rp < 4; ++rp)
             {
-                if (g + NG - 2 < ngroups) gp_wait_vmcnt<(NG - 2) * NV>();   // this wave's loads of group g landed
-                else gp_wait_vmcnt<0>();
-                gp_barrier();   // every wave's loads of group g landed; every wave is done with group g - 1
-                if (g + NG - 1 < ngroups) issue(g + NG - 1);   // into the slots of group g - 1
-                const uint8_t* sl = ring + (g % NG) * GB;
-                const uint16_t* xs = xring + (size_t)(g % NG) * GP_MT * GP_XS;
+                // the trellis words of this pair of tile rows (the next pair's reads go out under this decode)
+                uint32_t wd[GP_CPW][2][2];
 #pragma unroll
-                for (int rp = 0; rp < 4; ++rp)
-                {
-                    // the trellis words of this pair of tile rows (the next pair's reads go out under this decode)
-                    uint32_t wd[GP_CPW][2][2];
+                for (int c = 0; c < GP_CPW; ++c)
 #pragma unroll
-                    for (int c = 0; c < GP_CPW; ++c)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                        {
-                            const uint8_t* tp = sl + (2 * rp + h) * RB + c * TB;
-                            wd[c][h][0] = *reinterpret_cast<const uint32_t*>(tp + d.o0);
-                            wd[c][h][1] = *reinterpret_cast<const uint32_t*>(tp + d.o1);
-                        }
-                    half8 A[NMB];
-#pragma unroll
-                    for (int mb = 0; mb < NMB; ++mb)
-                        A[mb] = *reinterpret_cast<const half8*>(xs + (mb * 16 + i16) * GP_XS + q * 32 + rp * 8);
-                    half8 B[GP_CPW];
-#pragma unroll
-                    for (int c = 0; c < GP_CPW; ++c)
+                    for (int h = 0; h < 2; ++h)
                     {
-                        const half4 B0 = decode4<K>(wd[c][0][0], wd[c][0][1], d.sh);
-                        const half4 B1 = decode4<K>(wd[c][1][0], wd[c][1][1], d.sh);
-                        B[c] = half8{ B0[0], B0[1], B0[2], B0[3], B1[0], B1[1], B1[2], B1[3] };
+                        const uint8_t* tp = sl + (2 * rp + h) * RB + c * TB;
+                        wd[c][h][0] = *reinterpret_cast<const uint32_t*>(tp + d.o0);
+                        wd[c][h][1] = *reinterpret_cast<const uint32_t*>(tp + d.o1);
                     }
-                    // raised wave priority while this wave issues its MFMAs: the matrix pipe is refilled as soon as
-                    // it frees, and the other waves of the SIMD take the VALU slots in between
-                    __builtin_amdgcn_s_setprio(1);
+                half8 A[NMB];
 #pragma unroll
-                    for (int mb = 0; mb < NMB; ++mb)
+                for (int mb = 0; mb < NMB; ++mb)
+                    A[mb] = *reinterpret_cast<const half8*>(xs + (mb * 16 + i16) * GP_XS + q * 32 + rp * 8);
+                half8 B[GP_CPW];
 #pragma unroll
-                        for (int c = 0; c < GP_CPW; ++c)
-                            acc[c][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[mb], B[c], acc[c][mb], 0, 0, 0);
-                    __builtin_amdgcn_s_setprio(0);
+                for (int c = 0; c < GP_CPW; ++c)
+                {
+                    const half4 B0 = decode4<K>(wd[c][0][0], wd[c][0][1], d.sh);
+                    const half4 B1 = decode4<K>(wd[c][1][0], wd[c][1][1], d.sh);
+                    B[c] = half8{ B0[0], B0[1], B0[2], B0[3], B1[0], B1[1], B1[2], B1[3] };
                 }
-            }
-            // D[i][n]: lane holds rows 4q + rr of each 16-slot block, column (t0 + c) * 16 + i16
-#pragma unroll
-            for (int c = 0; c < GP_CPW; ++c)
+                // raised wave priority while this wave issues its MFMAs: the matrix pipe is refilled as soon as
+                // it frees, and the other waves of the SIMD take the VALU slots in between
+                __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                 for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
-                    for (int rr = 0; rr < 4; ++rr)
-                    {
-                        const int sl = mb * 16 + q * 4 + rr;
-                        if (sl < T)
-                            yout[(size_t)(c0 + sl) * a.ndim + (t0 + c) * 16 + i16] = (uint16_t)f2h_bits(acc[c][mb][rr]);
-                    }
-        };
-        static_assert(GP_MT == 80, "one case per row-block count");
-        switch ((T + 15) / 16)
-        {
-            case 1: pass(std::integral_constant<int, 1>{}); break;
-            case 2: pass(std::integral_constant<int, 2>{}); break;
-            case 3: pass(std::integral_constant<int, 3>{}); break;
-            case 4: pass(std::integral_constant<int, 4>{}); break;
-            default: pass(std::integral_constant<int, 5>{}); break;
+                    for (int c = 0; c < GP_CPW; ++c)
+                        acc[c][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[mb], B[c], acc[c][mb], 0, 0, 0);
+                __builtin_amdgcn_s_setprio(0);
+            }
         }
+        // D[i][n]: lane holds rows 4q + rr of each 16-slot block, column (t0 + c) * 16 + i16
+#pragma unroll
+        for (int c = 0; c < GP_CPW; ++c)
+#pragma unroll
+            for (int mb = 0; mb < NMB; ++mb)
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr)
+                {
+                    const int sl = mb * 16 + q * 4 + rr;
+                    if (sl < T)
+                        yout[(size_t)(c0 + sl) * a.ndim + (t0 + c) * 16 + i16] = (uint16_t)f2h_bits(acc[c][mb][rr]);
+                }
+    };
+    static_assert(GP_MT == 80, "one case per row-block count");
+    switch ((T + 15) / 16)
+    {
+        case 1: pass(std::integral_constant<int, 1>{}); break;
+        case 2: pass(std::integral_constant<int, 2>{}); break;
+        case 3: pass(std::integral_constant<int, 3>{}); break;
+        case 4: pass(std::integral_constant<int, 4>{}); break;
+        default: pass(std::integral_constant<int, 5>{}); break;
     }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// EXACT at prefill sizes: the reference's accumulator chains, each weight decoded once per pass of up to 64 slots
+// EXACT for many slots: the reference's accumulator chains, each weight decoded once per pass of an expert's slots
 // ---------------------------------------------------------------------------------------------------------------
 //
 // The reference's EXACT sum (tile_accum<M,EXACT>, ft_core.h:313-345) gives every output column n four fp32
@@ -671,89 +799,78 @@ __global__ __launch_bounds__(GP_NW * 64) void gp_gemm_kernel(GemmArgs a)
 // Here each chain step runs on the matrix cores. v_mfma_f32_16x16x1_4b_f32 computes four independent 16x16 rank-1
 // updates D_b = C_b + A_b B_b^T with K = 1. Per element that is one product added to one accumulator, and both
 // operands are fp16 values, so the product is exact in fp32 and D = RN(C + A B) = fmaf(A, B, C), the reference's
-// chain step. A probe on MI355X matched fmaf bit for bit on 4,096,000 elements (zeros, signed zeros and near-cancelling
-// sums included). Block b is chain j = b:
-//   - B: lane 16j + n holds chain j's weight of column n at step q. A lane decodes exactly the four weights its chain
-//     needs from each tile (stream indices 32 (n % 8) + 4 (n / 8) + j + 8q of the tile's stream, a3/PERM), and each
-//     decoded weight serves all the pass's slots.
-//   - A: lane 16j + m holds slot m's input for chain j at step q, x[slot][tk * 16 + 2q + off_j] (the input layout of
-//     xg_store_row): one ds_read_b128 per lane gives q = 0..3.
-//   - D: chain j of (slot 4 (l / 16) + i, column l % 16) sits in register 4j + i of lane l. The reduction
-//     (a0 + a1) + (a2 + a3) is then four registers of one lane.
-// A wave takes one tile column (16 outputs) with its 4 chains for every slot of the pass, in blocks of 16 slots (one
-// MFMA per block and step). Every accumulator is one chain of fused multiply-adds in the reference's order, so the
-// results are bit-identical to the decode path's.
+// chain step. v_mfma_f32_4x4x1_16b_f32 does the same for sixteen 4x4 blocks. Probes on MI355X matched both with fmaf bit
+// for bit on millions of elements (zeros, signed zeros and near-cancelling sums included).
+//   - Weights: a lane decodes four consecutive stream indices of a tile (decode4: column n, step q, chains 0..3), as the
+//     decode kernels do, and the transposing fp16 MFMA (a 0/1 permutation, exact) turns them into chain j's four steps of
+//     column n in lane 16j + n, as fp32. Decoding the lane's own four steps from four windows instead took 8 LDS reads and
+//     22 VALU instructions per tile (four funnel shifts, four conversions to fp32) against 2 and 15, and no fp32 MFMA
+//     hides VALU issue. With the groups of four below: M = 2048 layer 8.26 -> 7.36 ms, M = 333 2.42 -> 2.08 ms.
+//   - Whole blocks of 16 slots, 16x16x1: B is the weight register, A lane 16j + m holds slot m's input for chain j at
+//     step q (one ds_read_b128 per lane gives q = 0..3); chain j of (slot 4 (l / 16) + i, column l % 16) is register
+//     4j + i of lane l, and the reduction is four registers of one lane.
+//   - The slots past them: groups of four by 4x4x1 with the same two registers (cbsz = 2, abid = s: each chain's four
+//     blocks of 4 columns take A from its slots 4s..4s+3), then up to two single slots as v_fmac_f32 chains. A group
+//     costs 37 cycles of the SIMD per tile, a single slot 12 and a block of 16 128: a remainder of 13 to 15 slots is a
+//     padded block, 3, 7 and 11 are padded groups. Each remainder has a loop of its own: with the groups and single
+//     slots under branches inside one loop, the reads and decodes of a tile row could not move across them
+//     (M = 64 decode call 1151 -> 1087 us, M = 2048 7364 -> 7128 us).
+// A wave takes one tile column (16 outputs) with its 4 chains for every slot of the pass. Every accumulator is one chain
+// of fused multiply-adds in the reference's order, so the results are bit-identical to the decode path's.
+//
+// What bounds it: issue. Per tile about 80 cycles of VALU decode plus 8 cycles per slot of fp32 MFMA, which do not
+// overlap (the fp32 MFMA holds the SIMD's FMA units). At config 4 (M = 2048, 57 slots per expert) that sums to 6.4 ms
+// of the two GEMMs' 6.75 ms.
 
-// Waves per workgroup: 8 tile columns share one input ring. With the rings (76 KB of LDS at K=3) two workgroups fit
-// a CU, 4 waves per SIMD, which needs at most 128 VGPRs. Against 4-wave workgroups at 2 waves per SIMD this measured
-// 9.7 against 10.6 ms per config-4 layer.
-constexpr int XG_NW = 8;
+constexpr int XG_NW = 8;                    // waves per workgroup: 8 tile columns share one input ring
+constexpr int XG_MS = 64;                   // most slots per pass (xg_slots picks 16, 32 or 64 for a call)
 constexpr int XG_COLS = 16 * XG_NW;         // output columns per workgroup (a tile column per wave)
 constexpr int XG_TC = XG_COLS / 16;         // tile columns per workgroup
-constexpr int XG_MS = 64;                   // slots per pass
 constexpr int XG_NG = 2;                    // ring depth (groups of 8 tile rows)
 constexpr int XG_XROW = 8 * 16 * 4;         // input bytes of one slot per group: 8 tile rows x 16 rows x fp32
-constexpr int XG_XGB = XG_MS * XG_XROW;     // input bytes per group (32 KB)
-// Slots past a pass's whole blocks of 16 run as VALU chains when there are at most XG_REM of them, else as one more
-// MFMA block. A VALU chain slot costs a 16-byte LDS read and 4 v_fmac_f32 per tile row against a padded block's 4
-// MFMAs; at config 4 (about 57 slots per expert) thresholds 4, 6 and 8 measured 8.61, 8.60 and 8.70 ms per layer
-// against 8.95 ms with padding only.
-constexpr int XG_REM = 6;
 typedef float xg_acc __attribute__((ext_vector_type(16)));   // one 16-slot block of a wave's 4 x 16 x 16 accumulators
 
 struct XgArgs
 {
     const uint64_t* ptrs;
     int mat_base, nmat;        // first matrix of the launch (0 gate, 1 up, 2 down) and how many
-    int kdim, ndim, cap, E;
+    int kdim, ndim, cap, nit;  // nit: items the grid covers
     GPlan g;
     const float* xin;          // [mats][cap][kdim] fp32 (fp16-valued), accumulator-chain layout
     uint16_t* yout;            // [mats][cap][ndim] fp16: out_block's leading r16 (ft_core.h:109) applied here
 };
 
-// The 16-bit state of stream index t of a tile: the window of bits ending at (t + 1) K of the circular 256K-bit
-// stream (state_scalar, ft_core.h:65-73), as a funnel shift of two words (byte offsets o0, o1 in the tile) by sh.
-struct StateDec
+// Grid: 8 * ceil(items / 8) * (ndim / XG_COLS) * matrices, XCD-major as the MFMA GEMM. Workgroup = XG_NW waves x 16
+// columns (a tile column each, all 4 chains) of one matrix for one item, a pass of up to MS slots of an expert. Per group
+// of 8 tile rows the trellis of the XG_TC tile columns and the pass's inputs arrive by LDS-direct loads one group ahead
+// (one workgroup barrier per group); at the end each lane reduces its outputs' 4 chains.
+// Input rows are swizzled by the loads' source addresses: the 16-byte unit u of slot m's row chunk lands at unit
+// u ^ (m % 8), so that the 16 slots a fragment read takes at one unit lie in different banks (row stride 512 bytes).
+// Occupancy: the accumulators take MS VGPRs, so 16-, 32- and 64-slot passes fit 64, 80 and 128 registers (8, 6 and 4
+// waves per SIMD, 4, 3 and 2 workgroups per CU; their LDS fits too). With few slots the loop lives from other waves'
+// issue slots: M = 64 decode call, 16-slot passes at 6 and 8 waves 1087 and 1073 us, 32-slot ones at 4 and 6 waves 1263
+// and 1098 us.
+template <int K, int MS>
+__global__ __launch_bounds__(XG_NW * 64) __attribute__((amdgpu_waves_per_eu(MS >= 64 ? 4 : MS >= 32 ? 6 : 8))) void
+xg_gemm_kernel(XgArgs a)
 {
-    uint32_t o0, o1, sh;
-};
-__device__ __forceinline__ StateDec state_dec(int t, int K)
-{
-    const int e = (t + 1) * K, words = 8 * K;
-    const int wa = e >= 33 ? (e - 33) / 32 : -1;   // e - 32 wa in [33, 64]
-    StateDec d;
-    d.sh = (uint32_t)(64 - (e - 32 * wa));
-    d.o0 = (uint32_t)(4 * ((wa + words) % words));
-    d.o1 = (uint32_t)(4 * ((wa + 1 + words) % words));
-    return d;
-}
-
-
-// Grid: 8 * ceil(E / 8) * (ndim / XG_COLS) * matrices, XCD-major as the MFMA GEMM. Workgroup = XG_NW waves x 16
-// columns (a tile column each, all 4 chains) of one matrix of one expert; the expert's slots go through in passes of
-// XG_MS. Per group of 8 tile rows the trellis of the XG_TC tile columns and the pass's inputs arrive by LDS-direct
-// loads one group ahead (one workgroup barrier per group); at the end of a pass each lane reduces its outputs' 4
-// chains.
-template <int K>
-__global__ __launch_bounds__(XG_NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void xg_gemm_kernel(XgArgs a)
-{
-    constexpr int TB = 32 * K, RB = XG_TC * TB, GB = 8 * RB, NG = XG_NG;
+    constexpr int TB = 32 * K, RB = XG_TC * TB, GB = 8 * RB, NG = XG_NG, XGB = MS * XG_XROW;
     constexpr int NLD = GB / 256 / XG_NW;      // trellis dword loads per lane per group (the waves share a group)
+    constexpr int RPW = MS / XG_NW;            // input rows each wave loads per group
     static_assert(GB % (256 * XG_NW) == 0, "a group of tiles splits into whole loads of the waves");
     extern __shared__ __align__(16) uint8_t xg_lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nch = a.ndim / XG_COLS, per = nch * a.nmat;
     const int xcd = blockIdx.x % 8, jb = blockIdx.x / 8;
-    const int ei = (jb / per) * 8 + xcd, rr0 = jb % per;
-    if (ei >= a.E) return;
-    const int e = a.g.eord[ei];
+    const int it = (jb / per) * 8 + xcd, rr0 = jb % per;
+    if (it >= a.nit || it >= a.g.hdr[2]) return;
+    const int4 item = a.g.item[it];
+    const int e = item.x, c0 = item.y, T = item.z;
     const int nc = rr0 % nch;
     const int mat = a.mat_base + rr0 / nch;
-    const int s_begin = a.g.off[e], s_end = a.g.off[e + 1];
-    if (s_begin >= s_end) return;
     const int TN = a.ndim / 16, TK = a.kdim / 16, ngroups = TK / 8;
     uint8_t* tring = xg_lds;                                   // [NG][8 tile rows][XG_TC tile columns][TB]
-    uint8_t* xring = xg_lds + NG * GB;                         // [NG][XG_MS slots][8 tile rows][4 chains][4] fp32
+    uint8_t* xring = xg_lds + NG * GB;                         // [NG][MS slots][8 tile rows][4 chains][4] fp32, swizzled
     const uint8_t* tr = reinterpret_cast<const uint8_t*>(a.ptrs[(size_t)e * 9 + mat]);
     const int gs = TN * TB;                                    // bytes per tile row of the matrix
     uint8_t* cb = const_cast<uint8_t*>(uniform_ptr(tr + (size_t)nc * XG_TC * TB));
@@ -771,146 +888,173 @@ __global__ __launch_bounds__(XG_NW * 64) __attribute__((amdgpu_waves_per_eu(4)))
         const_cast<uint8_t*>(uniform_ptr(reinterpret_cast<const uint8_t*>(xin))), (short)0,
         (int)((size_t)a.cap * a.kdim * 4), 0x00020000);
     uint16_t* yout = a.yout + (size_t)(mat - a.mat_base) * a.cap * a.ndim;
-    // this lane's chain and column, and the stream windows of the chain's four weights in each tile
-    const int j = lane >> 4, tcl = wave, n = lane & 15;
-    StateDec sd[4];
+    // chain j of column n of the wave's tile column
+    const int j = lane >> 4, n = lane & 15;
+    const LaneDec d = lane_dec(lane, K);
+    half4 Pm;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) sd[q] = state_dec(32 * (n & 7) + 4 * (n >> 3) + j + 8 * q, K);
-    const int col0 = nc * XG_COLS;
+    for (int r = 0; r < 4; ++r) Pm[r] = (_Float16)((j == (n & 3) && r == (n >> 2)) ? 1.0f : 0.0f);
+    const float4v zero = { 0.f, 0.f, 0.f, 0.f };
+    // byte of unit 4 c + j (tile row c of 4, chain j) of slot n's row chunk, stored at unit (4 c + j) ^ (n % 8)
+    int xu[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) xu[c] = n * XG_XROW + (((4 * c + j) ^ (n & 7)) << 4);
 
-    for (int c0 = s_begin; c0 < s_end; c0 += XG_MS)
-    {
-        const int T = min(XG_MS, s_end - c0);
-        auto issue = [&](int g, int nsl) {
-            uint8_t* dst = tring + (g % NG) * GB;
+    auto issue = [&](int g, int nsl) {
+        uint8_t* dst = tring + (g % NG) * GB;
 #pragma unroll
-            for (int i = 0; i < NLD; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (gp_lds_void*)(dst + (wave * NLD + i) * 256), 4, voff[i],
-                                                         g * 8 * gs, 0, 0);
-            // this wave's RPW slot rows of the group (rows of slots past the pass repeat its last slot)
-            constexpr int RPW = XG_MS / XG_NW;
-            uint8_t* xd = xring + (g % NG) * XG_XGB;
-            if (wave * RPW < nsl)
+        for (int i = 0; i < NLD; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (gp_lds_void*)(dst + (wave * NLD + i) * 256), 4, voff[i],
+                                                     g * 8 * gs, 0, 0);
+        // this wave's RPW slot rows of the group (rows of slots past the pass repeat its last slot); the lane's source
+        // unit is permuted so that the row's 16-byte units land swizzled
+        uint8_t* xd = xring + (g % NG) * XGB;
+        if (wave * RPW < nsl)
+        {
+#pragma unroll
+            for (int r = 0; r < RPW; ++r)
             {
+                const int sl = wave * RPW + r;
+                const int srow = (c0 + min(sl, T - 1)) * a.kdim * 4 + g * XG_XROW;
+                const int vo = (((lane >> 2) ^ (sl & 7)) << 4) + (lane & 3) * 4;
 #pragma unroll
-                for (int r = 0; r < RPW; ++r)
-                {
-                    const int sl = wave * RPW + r;
-                    const int srow = (c0 + min(sl, T - 1)) * a.kdim * 4 + g * XG_XROW;
-#pragma unroll
-                    for (int h = 0; h < XG_XROW / 256; ++h)
-                        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (gp_lds_void*)(xd + sl * XG_XROW + h * 256), 4,
-                                                                 h * 256 + lane * 4, srow, 0, 0);
-                }
+                for (int h = 0; h < XG_XROW / 256; ++h)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (gp_lds_void*)(xd + sl * XG_XROW + h * 256), 4,
+                                                             h * 256 + vo, srow, 0, 0);
             }
-        };
-        // NSL slots in blocks of 16 on the matrix cores, then R <= XG_REM slots past them as VALU chains: lane
-        // (j, n) runs slot m's chain j of column n as v_fmac_f32 steps, fmaf(x, w, acc) as each K=1 MFMA step is, in
-        // the same step order, on the weights the lane decoded for the MFMAs
-        auto pass = [&](auto nsl_c, int R) {
-            constexpr int NSL = decltype(nsl_c)::value, NB = NSL / 16;
-            xg_acc acc[NB > 0 ? NB : 1];
+        }
+    };
+    // NB blocks of 16 slots, then NQ groups of 4 and NV single slots
+    auto pass = [&](auto nb_c, auto nq_c, auto nv_c) {
+        constexpr int NB = decltype(nb_c)::value, NQ = decltype(nq_c)::value, NV = decltype(nv_c)::value;
+        constexpr int NSL = 16 * NB;
+        xg_acc acc[NB > 0 ? NB : 1];
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
-            float racc[XG_REM];
+            for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+        float4v qacc[NQ > 0 ? NQ : 1];
+        float racc[NV > 0 ? NV : 1];
 #pragma unroll
-            for (int m = 0; m < XG_REM; ++m) racc[m] = 0.f;
-            __syncthreads();   // the previous pass is done with the rings
-            issue(0, NSL + R);
-            for (int g = 0; g < ngroups; ++g)
+        for (int m = 0; m < NQ; ++m) qacc[m] = zero;
+#pragma unroll
+        for (int m = 0; m < NV; ++m) racc[m] = 0.f;
+        issue(0, T);
+        for (int g = 0; g < ngroups; ++g)
+        {
+            gp_wait_vmcnt<0>();
+            gp_barrier();   // group g landed for every wave; every wave is done with group g - 1
+            if (g + 1 < ngroups) issue(g + 1, T);
+            const uint8_t* tl = tring + (g % NG) * GB + wave * TB;
+            const uint8_t* xl = xring + (g % NG) * XGB;
+#pragma unroll
+            for (int t8 = 0; t8 < 8; ++t8)
             {
-                gp_wait_vmcnt<0>();
-                gp_barrier();   // group g landed for every wave; every wave is done with group g - 1
-                if (g + 1 < ngroups) issue(g + 1, NSL + R);
-                const uint8_t* tl = tring + (g % NG) * GB + tcl * TB;
-                // lane (j, m) reads slot 16 b + m's inputs of chain j
-                const uint8_t* xl = xring + (g % NG) * XG_XGB + n * XG_XROW + j * 16;
-                // lane (j, n) reads remainder slot NSL + m's inputs of chain j (the same 16 bytes for all n)
-                const uint8_t* xr = xring + (g % NG) * XG_XGB + NSL * XG_XROW + j * 16;
+                const uint8_t* tp = tl + t8 * RB;
+                const uint32_t hi = *reinterpret_cast<const uint32_t*>(tp + d.o0);
+                const uint32_t lo = *reinterpret_cast<const uint32_t*>(tp + d.o1);
+                const float4v w = __builtin_amdgcn_mfma_f32_16x16x16f16(Pm, decode4<K>(hi, lo, d.sh), zero, 0, 0, 0);
+                const uint8_t* xt = xl + (t8 >> 2) * 256 + xu[t8 & 3];
+                float4 xv[NB > 0 ? NB : 1];
 #pragma unroll
-                for (int t8 = 0; t8 < 8; ++t8)
+                for (int b = 0; b < NB; ++b) xv[b] = *reinterpret_cast<const float4*>(xt + b * 16 * XG_XROW);
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[b].x, w[0], acc[b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[b].y, w[1], acc[b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[b].z, w[2], acc[b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[b].w, w[3], acc[b], 0, 0, 0);
+                if constexpr (NQ > 0)
                 {
-                    const uint8_t* tp = tl + t8 * RB;
-                    uint32_t st[4];
+                    const float4 xq = *reinterpret_cast<const float4*>(xt + NSL * XG_XROW);
+                    const float xs[4] = { xq.x, xq.y, xq.z, xq.w };
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
                     {
-                        const uint32_t hi = *reinterpret_cast<const uint32_t*>(tp + sd[q].o0);
-                        const uint32_t lo = *reinterpret_cast<const uint32_t*>(tp + sd[q].o1);
-                        st[q] = __builtin_amdgcn_alignbit(hi, lo, sd[q].sh) & 0xFFFFu;
-                    }
-                    const half4 wh = codebook4(st[0], st[1], st[2], st[3]);
-                    const float w[4] = { (float)wh[0], (float)wh[1], (float)wh[2], (float)wh[3] };
-                    float4 xv[NB > 0 ? NB : 1];
-#pragma unroll
-                    for (int b = 0; b < NB; ++b)
-                        xv[b] = *reinterpret_cast<const float4*>(xl + b * 16 * XG_XROW + t8 * 64);
-                    // steps q = 0..3 of the tile row; the blocks' chains are independent between dependent steps
-#pragma unroll
-                    for (int b = 0; b < NB; ++b)
-                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[b].x, w[0], acc[b], 0, 0, 0);
-#pragma unroll
-                    for (int b = 0; b < NB; ++b)
-                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[b].y, w[1], acc[b], 0, 0, 0);
-#pragma unroll
-                    for (int b = 0; b < NB; ++b)
-                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[b].z, w[2], acc[b], 0, 0, 0);
-#pragma unroll
-                    for (int b = 0; b < NB; ++b)
-                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[b].w, w[3], acc[b], 0, 0, 0);
-                    if (R > 0)
-                    {
-#pragma unroll
-                        for (int m = 0; m < XG_REM; ++m)
-                            if (m < R)
-                            {
-                                const float4 x4 = *reinterpret_cast<const float4*>(xr + m * XG_XROW + t8 * 64);
-                                racc[m] = __builtin_fmaf(x4.x, w[0], racc[m]);
-                                racc[m] = __builtin_fmaf(x4.y, w[1], racc[m]);
-                                racc[m] = __builtin_fmaf(x4.z, w[2], racc[m]);
-                                racc[m] = __builtin_fmaf(x4.w, w[3], racc[m]);
-                            }
+                        qacc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(xs[q], w[q], qacc[0], 2, 0, 0);
+                        if constexpr (NQ > 1)
+                            qacc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(xs[q], w[q], qacc[1], 2, 1, 0);
+                        if constexpr (NQ > 2)
+                            qacc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(xs[q], w[q], qacc[2], 2, 2, 0);
                     }
                 }
-            }
-            // chain c of (slot 16 b + 4 (lane / 16) + i, column lane % 16) is register 4c + i of acc[b]: the
-            // reference's (a0 + a1) + (a2 + a3), rounded to fp16 (out_block's leading r16)
-            const int col = col0 + tcl * 16 + n;
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int m = 0; m < NV; ++m)
                 {
-                    const int s = 16 * b + 4 * j + i;
-                    const float y = (acc[b][i] + acc[b][4 + i]) + (acc[b][8 + i] + acc[b][12 + i]);
-                    if (s < T) yout[(size_t)(c0 + s) * a.ndim + col] = (uint16_t)f2h_bits(y);
+                    constexpr int S0 = NSL + 4 * NQ;
+                    const float4 x4 = *reinterpret_cast<const float4*>(
+                        xl + (t8 >> 2) * 256 + (S0 + m) * XG_XROW + (((4 * (t8 & 3) + j) ^ ((S0 + m) & 7)) << 4));
+                    racc[m] = __builtin_fmaf(x4.x, w[0], racc[m]);
+                    racc[m] = __builtin_fmaf(x4.y, w[1], racc[m]);
+                    racc[m] = __builtin_fmaf(x4.z, w[2], racc[m]);
+                    racc[m] = __builtin_fmaf(x4.w, w[3], racc[m]);
                 }
-            // remainder slots: chain j of (slot, column n) is racc in lane 16 j + n
-            if (R > 0)
-            {
-#pragma unroll
-                for (int m = 0; m < XG_REM; ++m)
-                    if (m < R)
-                    {
-                        const float a1 = __shfl(racc[m], n + 16), a2 = __shfl(racc[m], n + 32),
-                                    a3 = __shfl(racc[m], n + 48);
-                        const float y = (racc[m] + a1) + (a2 + a3);
-                        if (j == 0) yout[(size_t)(c0 + NSL + m) * a.ndim + col] = (uint16_t)f2h_bits(y);
-                    }
             }
-        };
-        // slots past the last whole block of 16: up to XG_REM of them as VALU chains, more as one more MFMA block
-        const int R = T % 16 <= XG_REM ? T % 16 : 0;
-        switch ((T - R + 15) / 16)
-        {
-            case 0: pass(std::integral_constant<int, 0>{}, R); break;
-            case 1: pass(std::integral_constant<int, 16>{}, R); break;
-            case 2: pass(std::integral_constant<int, 32>{}, R); break;
-            case 3: pass(std::integral_constant<int, 48>{}, R); break;
-            default: pass(std::integral_constant<int, 64>{}, 0); break;
         }
+        // chain c of (slot 16 b + 4 (lane / 16) + i, column lane % 16) is register 4c + i of acc[b]: the
+        // reference's (a0 + a1) + (a2 + a3), rounded to fp16 (out_block's leading r16)
+        const int col = nc * XG_COLS + wave * 16 + n;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                const int s = 16 * b + 4 * j + i;
+                const float y = (acc[b][i] + acc[b][4 + i]) + (acc[b][8 + i] + acc[b][12 + i]);
+                if (s < T) yout[(size_t)(c0 + s) * a.ndim + col] = (uint16_t)f2h_bits(y);
+            }
+        auto put = [&](float v, int s) {
+            const float a1 = __shfl(v, n + 16), a2 = __shfl(v, n + 32), a3 = __shfl(v, n + 48);
+            const float y = (v + a1) + (a2 + a3);
+            if (j == 0 && s < T) yout[(size_t)(c0 + s) * a.ndim + col] = (uint16_t)f2h_bits(y);
+        };
+#pragma unroll
+        for (int m = 0; m < NQ; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) put(qacc[m][i], NSL + 4 * m + i);
+#pragma unroll
+        for (int m = 0; m < NV; ++m) put(racc[m], NSL + 4 * NQ + m);
+    };
+    // T slots: nb whole blocks of 16, then a remainder of R <= 12 as groups of four and single slots (13 to 15 fill
+    // one more block)
+    const int R = T % 16 > 12 ? 0 : T % 16, nb = (T - R + 15) / 16;
+    auto n0 = std::integral_constant<int, 0>{};
+    auto n1 = std::integral_constant<int, 1>{};
+    auto n2 = std::integral_constant<int, 2>{};
+    auto n3 = std::integral_constant<int, 3>{};
+    auto rest = [&](auto nb_c) {
+        switch (R)
+        {
+            case 0:
+                if constexpr (decltype(nb_c)::value > 0) pass(nb_c, n0, n0);
+                break;
+            case 1: pass(nb_c, n0, n1); break;
+            case 2: pass(nb_c, n0, n2); break;
+            case 3:
+            case 4: pass(nb_c, n1, n0); break;
+            case 5: pass(nb_c, n1, n1); break;
+            case 6: pass(nb_c, n1, n2); break;
+            case 7:
+            case 8: pass(nb_c, n2, n0); break;
+            case 9: pass(nb_c, n2, n1); break;
+            case 10: pass(nb_c, n2, n2); break;
+            default: pass(nb_c, n3, n0); break;
+        }
+    };
+    if (nb == MS / 16) pass(std::integral_constant<int, MS / 16>{}, n0, n0);
+    else if (nb == 0) rest(n0);
+    if constexpr (MS > 16)
+        if (nb == 1) rest(n1);
+    if constexpr (MS > 32)
+    {
+        if (nb == 2) rest(n2);
+        else if (nb == 3) rest(n3);
     }
 }
 
@@ -934,7 +1078,7 @@ static int gp_gemm_launch(const GemmArgs& a, int nmat, hipStream_t st)
     if (!opened) return -1;
     GemmArgs b = a;
     b.nmat = nmat;
-    const unsigned grid = (unsigned)(((a.E + 7) / 8) * 8 * (a.ndim / GP_WCOLS) * nmat);
+    const unsigned grid = (unsigned)(((a.nit + 7) / 8) * 8 * (a.ndim / GP_WCOLS) * nmat);
     hipLaunchKernelGGL(gp_gemm_kernel<K>, dim3(grid), dim3(GP_NW * 64), lds, st, b);
     return 0;
 }
@@ -951,47 +1095,96 @@ static int gp_gemm(int K, const GemmArgs& a, int nmat, hipStream_t st)
     }
 }
 
-template <int K>
-static size_t xg_gemm_lds()
-{
-    return (size_t)XG_NG * 8 * XG_TC * 32 * K + (size_t)XG_NG * XG_XGB;
-}
-
-template <int K>
+template <int K, int MS>
 static int xg_gemm_launch(const XgArgs& a, int nmat, hipStream_t st)
 {
-    const size_t lds = xg_gemm_lds<K>();
-    static const bool opened = hipFuncSetAttribute(reinterpret_cast<const void*>(xg_gemm_kernel<K>),
+    constexpr size_t lds = (size_t)XG_NG * 8 * XG_TC * 32 * K + (size_t)XG_NG * MS * XG_XROW;
+    static const bool opened = hipFuncSetAttribute(reinterpret_cast<const void*>(xg_gemm_kernel<K, MS>),
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
     if (!opened) return -1;
     XgArgs b = a;
     b.nmat = nmat;
-    const unsigned grid = (unsigned)(((a.E + 7) / 8) * 8 * (a.ndim / XG_COLS) * nmat);
-    hipLaunchKernelGGL(xg_gemm_kernel<K>, dim3(grid), dim3(XG_NW * 64), lds, st, b);
+    const unsigned grid = (unsigned)(((a.nit + 7) / 8) * 8 * (a.ndim / XG_COLS) * nmat);
+    hipLaunchKernelGGL((xg_gemm_kernel<K, MS>), dim3(grid), dim3(XG_NW * 64), lds, st, b);
     return 0;
 }
 
-static int xg_gemm(int K, const XgArgs& a, int nmat, hipStream_t st)
+// Slots per pass of a call of P picks over E experts: the smallest pass that holds an expert's mean share, since a
+// smaller pass leaves more waves per SIMD and a larger one decodes an expert's weights less often. Measured at E = 288,
+// top-8 (ms per layer with 16 / 32 / 64; P / E in brackets): M = 64 [1.8] 1.05 / 1.07 / 1.27, M = 333 [9.3] 1.62 / 1.64 /
+// 1.80, M = 500 [14] 2.75 / 2.59 / 2.77, M = 700 [19] 3.71 / 3.12 / 3.35, M = 1024 [28] 5.05 / 4.21 / 4.22, M = 2048 [57]
+// 9.39 / 7.84 / 7.07.
+static int xg_slots(int P, int E)
+{
+    return P < 8 * E ? 16 : P < 28 * E ? 32 : XG_MS;
+}
+
+template <int K>
+static int xg_gemm_k(int ms, const XgArgs& a, int nmat, hipStream_t st)
+{
+    return ms == 16   ? xg_gemm_launch<K, 16>(a, nmat, st)
+           : ms == 32 ? xg_gemm_launch<K, 32>(a, nmat, st)
+                      : xg_gemm_launch<K, XG_MS>(a, nmat, st);
+}
+
+static int xg_gemm(int K, int ms, const XgArgs& a, int nmat, hipStream_t st)
 {
     switch (K)
     {
-        case 2: return xg_gemm_launch<2>(a, nmat, st);
-        case 3: return xg_gemm_launch<3>(a, nmat, st);
-        case 4: return xg_gemm_launch<4>(a, nmat, st);
-        case 5: return xg_gemm_launch<5>(a, nmat, st);
+        case 2: return xg_gemm_k<2>(ms, a, nmat, st);
+        case 3: return xg_gemm_k<3>(ms, a, nmat, st);
+        case 4: return xg_gemm_k<4>(ms, a, nmat, st);
+        case 5: return xg_gemm_k<5>(ms, a, nmat, st);
         default: return -1;
     }
 }
 
-void launch_grouped_plan(const int64_t* sel, const void* w, int w_half, int P, int topk, int E, const GPlan& g,
-                         hipStream_t st)
+void launch_grouped_plan(const uint64_t* ptrs, const int64_t* sel, const void* w, int w_half, int P, int topk, int E,
+                         int mt, const GPlan& g, hipStream_t st)
 {
     const int M = P / topk;
     const unsigned nch = (unsigned)((P + GP_PLAN_CHUNK - 1) / GP_PLAN_CHUNK);
+    if (nch == 1)
+    {
+        hipLaunchKernelGGL(gp_plan_kernel, dim3(1), dim3(GP_PLAN_THREADS), 0, st, ptrs, sel, w, w_half, P, topk, E, mt, g);
+        return;
+    }
     hipLaunchKernelGGL(gp_rank_kernel, dim3(nch), dim3(GP_PLAN_THREADS), 0, st, sel, P, E, g);
-    hipLaunchKernelGGL(gp_place_kernel, dim3(nch), dim3(GP_PLAN_THREADS), 0, st, sel, P, E, g);
+    hipLaunchKernelGGL(gp_place_kernel, dim3(nch), dim3(GP_PLAN_THREADS), 0, st, sel, P, E, mt, g);
     hipLaunchKernelGGL(gp_order_kernel, dim3((unsigned)((M + GP_ORDER_THREADS - 1) / GP_ORDER_THREADS)),
-                       dim3(GP_ORDER_THREADS), 0, st, w, w_half, M, topk, g);
+                       dim3(GP_ORDER_THREADS), 0, st, ptrs, w, w_half, M, topk, g);
+}
+
+// Waves per slot of the input transform: one where the slots alone make about 4 waves per SIMD, else up to one per chunk
+// of blocks.
+static int prep_parts(int P, int H)
+{
+    const int most = (H / 128 + 4 * GP_TU - 1) / (4 * GP_TU);
+    return std::max(1, std::min(most, 4096 / P));
+}
+
+template <bool XL, int TA>
+static void act_launch_ta(const uint64_t* ptrs, int P, int I, int cap, const GPlan& g, const uint16_t* ygu,
+                          const float* silu_tab, float act_limit, void* xd, hipStream_t st)
+{
+    const long items = (long)P * ((I / 128 + 4 * TA - 1) / (4 * TA));
+    hipLaunchKernelGGL((gp_act_kernel<XL, TA>), dim3((unsigned)((items + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
+                       ptrs, I, cap, g, ygu, silu_tab, act_limit, xd);
+}
+
+template <bool XL>
+static void act_launch(const uint64_t* ptrs, int P, int I, int cap, const GPlan& g, const uint16_t* ygu,
+                       const float* silu_tab, float act_limit, void* xd, hipStream_t st)
+{
+    if (P <= GP_SMALL) act_launch_ta<XL, 1>(ptrs, P, I, cap, g, ygu, silu_tab, act_limit, xd, st);
+    else act_launch_ta<XL, GP_TA>(ptrs, P, I, cap, g, ygu, silu_tab, act_limit, xd, st);
+}
+
+static void comb_launch(int H, int M, int topk, const GPlan& g, const uint16_t* yraw, float* out, hipStream_t st)
+{
+    const long items = (long)M * ((H / 128 + 3) / 4);
+    hipLaunchKernelGGL(gp_comb_kernel, dim3((unsigned)((items + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st, H, M,
+                       topk, g, yraw, out);
 }
 
 int launch_grouped(const uint64_t* ptrs, const int64_t* sel, const void* w, int w_half, int P, int topk, int E, int H,
@@ -1000,12 +1193,13 @@ int launch_grouped(const uint64_t* ptrs, const int64_t* sel, const void* w, int 
                    hipStream_t st)
 {
     const int M = P / topk;
-    launch_grouped_plan(sel, w, w_half, P, topk, E, g, st);
-    const unsigned slot_wgs = (unsigned)((P + GP_TW - 1) / GP_TW);
-    hipLaunchKernelGGL(gp_prep_kernel<false>, dim3(slot_wgs), dim3(GP_TW * 64), 0, st, ptrs, x, H, topk, cap, g,
+    launch_grouped_plan(ptrs, sel, w, w_half, P, topk, E, GP_MT, g, st);
+    const int parts = prep_parts(P, H);
+    hipLaunchKernelGGL(gp_prep_kernel<false>, dim3((unsigned)(((long)P * parts + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
+                       ptrs, x, H, topk, cap, parts, g,
                        static_cast<void*>(xt));
     GemmArgs a;
-    a.ptrs = ptrs; a.kdim = H; a.ndim = I; a.cap = cap; a.E = E; a.g = g; a.xin = xt; a.yout = ygu;
+    a.ptrs = ptrs; a.kdim = H; a.ndim = I; a.cap = cap; a.nit = gemm_items(P, E, GP_MT); a.g = g; a.xin = xt; a.yout = ygu;
     if (Kg == Ku)
     {
         a.mat_base = 0;
@@ -1021,17 +1215,11 @@ int launch_grouped(const uint64_t* ptrs, const int64_t* sel, const void* w, int 
         b.yout = ygu + (size_t)cap * I;
         if (gp_gemm(Ku, b, 1, st)) return -1;
     }
-    const long act_items = (long)P * ((I / 128 + 4 * GP_TA - 1) / (4 * GP_TA));
-    hipLaunchKernelGGL(gp_act_kernel<false>, dim3((unsigned)((act_items + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0,
-                       st, ptrs, I, cap, g, ygu, silu_tab, act_limit, static_cast<void*>(xd));
+    act_launch<false>(ptrs, P, I, cap, g, ygu, silu_tab, act_limit, xd, st);
     GemmArgs c = a;
     c.mat_base = 2; c.kdim = I; c.ndim = H; c.xin = xd; c.yout = yraw;
     if (gp_gemm(Kd, c, 1, st)) return -1;
-    {
-        const long items = (long)M * ((H / 128 + 3) / 4);
-        hipLaunchKernelGGL(gp_comb_kernel, dim3((unsigned)((items + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st, ptrs,
-                           H, M, topk, g, yraw, out);
-    }
+    comb_launch(H, M, topk, g, yraw, out, st);
     return 0;
 }
 
@@ -1043,38 +1231,34 @@ int launch_exact_chains(const uint64_t* ptrs, const int64_t* sel, const void* w,
     // the chain GEMM addresses its fp32 inputs with 32-bit byte offsets
     if ((size_t)cap * (size_t)(H > I ? H : I) * 4 > (size_t)0x7fffffff) return -1;
     const int M = P / topk;
-    launch_grouped_plan(sel, w, w_half, P, topk, E, g, st);
-    const unsigned slot_wgs = (unsigned)((P + GP_TW - 1) / GP_TW);
-    hipLaunchKernelGGL(gp_prep_kernel<true>, dim3(slot_wgs), dim3(GP_TW * 64), 0, st, ptrs, x, H, topk, cap, g,
+    const int ms = xg_slots(P, E);
+    launch_grouped_plan(ptrs, sel, w, w_half, P, topk, E, ms, g, st);
+    const int parts = prep_parts(P, H);
+    hipLaunchKernelGGL(gp_prep_kernel<true>, dim3((unsigned)(((long)P * parts + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
+                       ptrs, x, H, topk, cap, parts, g,
                        static_cast<void*>(xt));
     XgArgs a;
-    a.ptrs = ptrs; a.kdim = H; a.ndim = I; a.cap = cap; a.E = E; a.g = g; a.xin = xt; a.yout = ygu;
+    a.ptrs = ptrs; a.kdim = H; a.ndim = I; a.cap = cap; a.nit = gemm_items(P, E, ms); a.g = g; a.xin = xt; a.yout = ygu;
     if (Kg == Ku)
     {
         a.mat_base = 0;
-        if (xg_gemm(Kg, a, 2, st)) return -1;
+        if (xg_gemm(Kg, ms, a, 2, st)) return -1;
     }
     else
     {
         a.mat_base = 0;
-        if (xg_gemm(Kg, a, 1, st)) return -1;
+        if (xg_gemm(Kg, ms, a, 1, st)) return -1;
         XgArgs b = a;
         b.mat_base = 1;
         b.xin = xt + (size_t)cap * H;
         b.yout = ygu + (size_t)cap * I;
-        if (xg_gemm(Ku, b, 1, st)) return -1;
+        if (xg_gemm(Ku, ms, b, 1, st)) return -1;
     }
-    const long act_items = (long)P * ((I / 128 + 4 * GP_TA - 1) / (4 * GP_TA));
-    hipLaunchKernelGGL(gp_act_kernel<true>, dim3((unsigned)((act_items + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0,
-                       st, ptrs, I, cap, g, ygu, silu_tab, act_limit, static_cast<void*>(xd));
+    act_launch<true>(ptrs, P, I, cap, g, ygu, silu_tab, act_limit, xd, st);
     XgArgs c = a;
     c.mat_base = 2; c.kdim = I; c.ndim = H; c.xin = xd; c.yout = yraw;
-    if (xg_gemm(Kd, c, 1, st)) return -1;
-    {
-        const long items = (long)M * ((H / 128 + 3) / 4);
-        hipLaunchKernelGGL(gp_comb_kernel, dim3((unsigned)((items + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st, ptrs,
-                           H, M, topk, g, yraw, out);
-    }
+    if (xg_gemm(Kd, ms, c, 1, st)) return -1;
+    comb_launch(H, M, topk, g, yraw, out, st);
     return 0;
 }
 
