@@ -578,6 +578,8 @@ int gfl_ctx_destroy(gfl_ctx* c)
     return GFL_OK;
 }
 
+static int reserve_chains(gfl_ctx* c, const Layer& L);
+
 int gfl_register_layer(gfl_ctx* c, int li, int E, int H, int I, int k_gate, int k_up, int k_down, const uint64_t* ptrs)
 {
     if (!c || !ptrs) return fail(GFL_EINVAL, "gfl_register_layer: NULL argument");
@@ -602,8 +604,9 @@ int gfl_register_layer(gfl_ctx* c, int li, int E, int H, int I, int k_gate, int 
     GFL_HIP(hipMemcpy(L.dptrs, ptrs, sizeof(uint64_t) * 9 * (size_t)E, hipMemcpyHostToDevice));
     L.E = E; L.H = H; L.I = I; L.K[0] = k_gate; L.K[1] = k_up; L.K[2] = k_down;
     L.shared = 0;
-    // the decode workspace for this shape, reserved now so that no forward call allocates
-    return reserve_ws(c, H, I);
+    // the workspaces of calls of up to MAX_PICKS picks for this shape, reserved now so that no such call allocates
+    if (const int r = reserve_ws(c, H, I)) return r;
+    return reserve_chains(c, L);
 }
 
 int gfl_register_shared(gfl_ctx* c, int li, int k_gate, int k_up, int k_down, const uint64_t* ptr_row)
@@ -636,8 +639,39 @@ int gfl_register_shared(gfl_ctx* c, int li, int k_gate, int k_up, int k_down, co
     return GFL_OK;
 }
 
-static int run_forward_grouped_plan(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64_t* sel, const void* w,
-                                    int w_is_half, int M, int topk, float* out, float act_limit, hipStream_t st);
+static int run_chains(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64_t* sel, const void* w, int w_is_half,
+                      int M, int topk, float* out, float act_limit, hipStream_t st);
+
+// Whether an EXACT call takes the accumulator-chain GEMMs on the grouped plan (run_chains) instead of the decode
+// launches: always above MAX_PICKS picks; below, from half a pick per expert on, three quarters where gate and up have
+// different bits and so a launch each (and above the 64 picks of the relay launches). The chain GEMM decodes an expert's weights once for all its slots, the decode launches once per 2 slots,
+// but it takes six launches instead of three. Measured (decode launches -> chains, us per layer, top-8; picks per expert in
+// brackets): E = 288, uniform routing: M = 9 [0.25] 261 -> 260, M = 16 [0.44] 420 -> 413, M = 24 [0.67] 600 -> 553, M = 64
+// [1.8] 1353 -> 1055; gate 3 and up 5 bits M = 18 [0.5] 515 -> 530, M = 27 [0.75] 705 -> 658; H=2048 I=768 M = 9 75 -> 82,
+// M = 16 117 -> 117, M = 24 153 -> 142, gate 3 up 5 bits M = 22 157 -> 165, M = 27 181 -> 177; E = 72: M = 9 [1] 259 -> 240, M = 64 [7.1] 1250 -> 526; Zipf 1.1 over 288: M = 16
+// 527 -> 329, M = 32 991 -> 445.
+// The chains' combine writes 16 bytes at a time, and the forced launch shapes (GFL_SLOTS_PER_PASS, GFL_RELAY) name the
+// decode launches, so an unaligned out and a context with either keep those.
+static bool takes_chains(const gfl_ctx* c, const Layer& L, int P, int mode, const float* out)
+{
+    if (mode == GFL_MODE_MFMA) return false;
+    if (P > gfl::MAX_PICKS) return true;
+    const bool enough = L.K[0] == L.K[1] ? 2 * P >= L.E : 4 * P >= 3 * L.E;
+    return P > 64 && enough && !(reinterpret_cast<uintptr_t>(out) & 15) && c->ns_override == 0 &&
+           c->rw_override[0] < 0;
+}
+
+// A call of picks on the launches that suit it (caller holds c->mu, device set; arguments checked).
+static int forward_picks(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64_t* sel, const void* w, int w_is_half,
+                         int M, int topk, float* out, int mode, float act_limit, hipStream_t st, const char* who)
+{
+    if (takes_chains(c, L, M * topk, mode, out))
+        return run_chains(c, L, x, sel, w, w_is_half, M, topk, out, act_limit, st);
+    if (!c->ws || L.H > c->ws_H || L.I > c->ws_I) return fail(GFL_ERUNTIME, std::string(who) + ": workspace not reserved");
+    Workspace ws;
+    carve_ws(c, L.H, L.I, ws);
+    return run_forward(c, L, ws, x, sel, w, w_is_half, M, topk, out, mode, act_limit, st, true);
+}
 
 int gfl_moe_forward(gfl_ctx* c, int li, const uint16_t* x, const int64_t* sel, const void* w, int w_is_half, int M,
                     int topk, float* out, int mode, float act_limit, gfl_stream stream)
@@ -650,14 +684,8 @@ int gfl_moe_forward(gfl_ctx* c, int li, const uint16_t* x, const int64_t* sel, c
     const Layer& L = c->layers[li];
     if (topk == 0) return forward_without_picks(c, L, M, out, reinterpret_cast<hipStream_t>(stream));
     GFL_HIP(hipSetDevice(c->device));
-    if (M * topk > gfl::MAX_PICKS)
-        return run_forward_grouped_plan(c, L, x, sel, w, w_is_half, M, topk, out, act_limit,
-                                        reinterpret_cast<hipStream_t>(stream));
-    if (!c->ws || L.H > c->ws_H || L.I > c->ws_I) return fail(GFL_ERUNTIME, "gfl_moe_forward: workspace not reserved");
-    Workspace ws;
-    carve_ws(c, L.H, L.I, ws);
-    return run_forward(c, L, ws, x, sel, w, w_is_half, M, topk, out, mode, act_limit,
-                       reinterpret_cast<hipStream_t>(stream), true);
+    return forward_picks(c, L, x, sel, w, w_is_half, M, topk, out, mode, act_limit,
+                         reinterpret_cast<hipStream_t>(stream), "gfl_moe_forward");
 }
 
 int gfl_moe_forward_shared(gfl_ctx* c, int li, const uint16_t* x, const int64_t* sel, const void* w, int w_is_half,
@@ -790,11 +818,18 @@ static int grouped_workspace(gfl_ctx* c, hipStream_t st, int P, int M, int E, in
     return GFL_OK;
 }
 
-// EXACT above MAX_PICKS picks (caller holds c->mu, device set): the grouped plan of the prefill path, then the
+// The prefill workspace for the chains at up to MAX_PICKS picks of layer L, so that such calls never allocate.
+static int reserve_chains(gfl_ctx* c, const Layer& L)
+{
+    Gws ws;
+    return grouped_workspace(c, nullptr, gfl::MAX_PICKS, gfl::MAX_PICKS, L.E, L.H, L.I, "gfl_register_layer", ws);
+}
+
+// EXACT on the accumulator chains (caller holds c->mu, device set): the grouped plan of the prefill path, then the
 // reference's accumulator chains with each weight decoded once per pass of up to 64 of an expert's slots
-// (launch_exact_chains, bit-identical to the decode path).
-static int run_forward_grouped_plan(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64_t* sel, const void* w,
-                                    int w_is_half, int M, int topk, float* out, float act_limit, hipStream_t st)
+// (launch_chains_*, bit-identical to the decode launches).
+static int run_chains(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64_t* sel, const void* w, int w_is_half,
+                      int M, int topk, float* out, float act_limit, hipStream_t st)
 {
     const int P = M * topk;
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) & 15)
@@ -803,11 +838,25 @@ static int run_forward_grouped_plan(gfl_ctx* c, const Layer& L, const uint16_t* 
         return fail(GFL_EINVAL, "gfl_moe_forward: M*topk*max(H, I) must stay below 2^29 above 1024 picks");
     Gws ws;
     if (const int rc = grouped_workspace(c, st, P, M, L.E, L.H, L.I, "gfl_moe_forward", ws)) return rc;
-    const int r = staged(c, 1, st, [&] {
-        return gfl::launch_exact_chains(L.dptrs, sel, w, w_is_half ? 1 : 0, P, topk, L.E, L.H, L.I, L.K[0], L.K[1],
-                                        L.K[2], x, ws.gp, P, ws.xte, ws.ygue, ws.xde, ws.yre, c->silu_tab, act_limit,
-                                        out, st);
-    });
+    auto gate_up = [&] {
+        return gfl::launch_chains_gate_up(L.dptrs, sel, w, w_is_half ? 1 : 0, P, topk, L.E, L.H, L.I, L.K[0], L.K[1], x,
+                                          ws.gp, P, ws.xte, ws.ygue, ws.xde, c->silu_tab, act_limit, st);
+    };
+    auto down = [&] {
+        return gfl::launch_chains_down(L.dptrs, P, topk, L.E, L.H, L.I, L.K[2], ws.gp, P, ws.xde, ws.yre, out, st);
+    };
+    // up to MAX_PICKS picks the stages are the decode launches' (1 gate|up, 3 down); above, the call is one stage
+    int r;
+    if (P <= gfl::MAX_PICKS)
+    {
+        r = staged(c, 1, st, gate_up);
+        if (!r) r = staged(c, 3, st, down);
+    }
+    else
+        r = staged(c, 1, st, [&] {
+            const int g = gate_up();
+            return g ? g : down();
+        });
     if (r) return r > 0 ? r : fail(GFL_EINVAL, "gfl_moe_forward: unsupported K or launch shape");
     GFL_HIP(hipGetLastError());
     c->calls += 1;
@@ -1056,13 +1105,10 @@ int gfl_ingress_serve(gfl_ctx* c, int li, int bsz, int topk, int64_t* ctrl, cons
     std::lock_guard<std::mutex> g(c->mu);
     const Layer& L = c->layers[li];
     GFL_HIP(hipSetDevice(c->device));
-    if (!c->ws || L.H > c->ws_H || L.I > c->ws_I) return fail(GFL_ERUNTIME, std::string(who) + ": workspace not reserved");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     gfl::launch_ingress_take(ctrl, hpicks, li, bsz, topk, L.E, c->ing_sel, c->ing_w, c->ing_state, c->status, st);
     GFL_HIP(hipGetLastError());
-    Workspace ws;
-    carve_ws(c, L.H, L.I, ws);
-    if (const int r = run_forward(c, L, ws, hx, c->ing_sel, c->ing_w, 0, bsz, topk, hout, mode, act_limit, st, true))
+    if (const int r = forward_picks(c, L, hx, c->ing_sel, c->ing_w, 0, bsz, topk, hout, mode, act_limit, st, who))
         return r;
     gfl::launch_ingress_answer(ctrl, c->ing_state, st);
     GFL_HIP(hipGetLastError());

@@ -1223,42 +1223,45 @@ int launch_grouped(const uint64_t* ptrs, const int64_t* sel, const void* w, int 
     return 0;
 }
 
-int launch_exact_chains(const uint64_t* ptrs, const int64_t* sel, const void* w, int w_half, int P, int topk, int E,
-                        int H, int I, int Kg, int Ku, int Kd, const uint16_t* x, const GPlan& g, int cap, float* xt,
-                        uint16_t* ygu, float* xd, uint16_t* yraw, const float* silu_tab, float act_limit, float* out,
-                        hipStream_t st)
+int launch_chains_gate_up(const uint64_t* ptrs, const int64_t* sel, const void* w, int w_half, int P, int topk, int E,
+                          int H, int I, int Kg, int Ku, const uint16_t* x, const GPlan& g, int cap, float* xt,
+                          uint16_t* ygu, float* xd, const float* silu_tab, float act_limit, hipStream_t st)
 {
     // the chain GEMM addresses its fp32 inputs with 32-bit byte offsets
     if ((size_t)cap * (size_t)(H > I ? H : I) * 4 > (size_t)0x7fffffff) return -1;
-    const int M = P / topk;
     const int ms = xg_slots(P, E);
     launch_grouped_plan(ptrs, sel, w, w_half, P, topk, E, ms, g, st);
     const int parts = prep_parts(P, H);
     hipLaunchKernelGGL(gp_prep_kernel<true>, dim3((unsigned)(((long)P * parts + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
-                       ptrs, x, H, topk, cap, parts, g,
-                       static_cast<void*>(xt));
+                       ptrs, x, H, topk, cap, parts, g, static_cast<void*>(xt));
     XgArgs a;
     a.ptrs = ptrs; a.kdim = H; a.ndim = I; a.cap = cap; a.nit = gemm_items(P, E, ms); a.g = g; a.xin = xt; a.yout = ygu;
+    a.mat_base = 0;
     if (Kg == Ku)
     {
-        a.mat_base = 0;
         if (xg_gemm(Kg, ms, a, 2, st)) return -1;
     }
     else
     {
-        a.mat_base = 0;
         if (xg_gemm(Kg, ms, a, 1, st)) return -1;
-        XgArgs b = a;
-        b.mat_base = 1;
-        b.xin = xt + (size_t)cap * H;
-        b.yout = ygu + (size_t)cap * I;
-        if (xg_gemm(Ku, ms, b, 1, st)) return -1;
+        a.mat_base = 1;
+        a.xin = xt + (size_t)cap * H;
+        a.yout = ygu + (size_t)cap * I;
+        if (xg_gemm(Ku, ms, a, 1, st)) return -1;
     }
     act_launch<true>(ptrs, P, I, cap, g, ygu, silu_tab, act_limit, xd, st);
-    XgArgs c = a;
-    c.mat_base = 2; c.kdim = I; c.ndim = H; c.xin = xd; c.yout = yraw;
-    if (xg_gemm(Kd, ms, c, 1, st)) return -1;
-    comb_launch(H, M, topk, g, yraw, out, st);
+    return 0;
+}
+
+int launch_chains_down(const uint64_t* ptrs, int P, int topk, int E, int H, int I, int Kd, const GPlan& g, int cap,
+                       const float* xd, uint16_t* yraw, float* out, hipStream_t st)
+{
+    const int ms = xg_slots(P, E);
+    XgArgs a;
+    a.ptrs = ptrs; a.mat_base = 2; a.kdim = I; a.ndim = H; a.cap = cap; a.nit = gemm_items(P, E, ms); a.g = g;
+    a.xin = xd; a.yout = yraw;
+    if (xg_gemm(Kd, ms, a, 1, st)) return -1;
+    comb_launch(H, P / topk, topk, g, yraw, out, st);
     return 0;
 }
 

@@ -95,8 +95,8 @@ int gfl_ctx_check(gfl_ctx* ctx);
  * (glm53/expert_cache.py:540-635). */
 int gfl_register_layer(gfl_ctx* ctx, int li, int E, int H, int I, int k_gate, int k_up, int k_down,
                        const uint64_t* ptrs);
-/* (Registration also reserves the decode workspace for 1024 picks at the largest registered H and I, so that
- * gfl_moe_forward never allocates.) */
+/* (Registration also reserves the decode and prefill workspaces for 1024 picks at the largest registered sizes, so that
+ * gfl_moe_forward never allocates up to 1024 picks.) */
 
 /* Shape of a registered layer: info[6] = {E, H, I, k_gate, k_up, k_down} (host array). The forward calls take no
  * shape arguments, so callers check their x / out widths against H with it (tier_forward checks x.size(1) == H,
@@ -110,12 +110,13 @@ int gfl_layer_info(gfl_ctx* ctx, int li, int* info);
  * act_limit: SwiGLU clamp (tier_set_act_limit, ft_tier_ext.cpp:629-636), 0 = off. topk <= 16; x 16-byte aligned.
  * Empty calls, as the reference's tier_forward takes them (ft_tier_ext.cpp:893-903): M = 0 does nothing (every
  * buffer may be NULL); topk = 0 writes M rows of zeros to out (sel and w may be NULL).
- * M*topk <= 1024: the decode launches (routing plan built in every workgroup). 1024 < M*topk <= 65536 (EXACT modes
- * only; MFMA is refused there): the grouped plan of the prefill path, then the reference's accumulator chains (each
- * chain step one element of a K=1 fp32 MFMA, i.e. an fmaf), each weight decoded once per pass of up to 64 of an
- * expert's slots, bit-identical to the reference's EXACT mode at any batch size; there out must be 16-byte aligned
- * too and M*topk*max(H, I) < 2^29. That path uses the prefill workspace (gfl_grouped_reserve sizes it ahead of graph
- * capture; otherwise the first call of a larger size grows it). */
+ * M*topk <= 64, and up to 1024 with fewer than half a pick per expert of the layer (three quarters where gate and up
+ * have different bits), mode MFMA or an out that is not 16-byte aligned: the decode launches. Other calls up to M*topk = 65536 (EXACT modes only; MFMA is refused above 1024):
+ * the grouped plan of the prefill path, then the reference's accumulator chains (each chain step one element of a K=1
+ * fp32 MFMA, i.e. an fmaf), each weight decoded once per pass of up to 64 of an expert's slots, bit-identical to the
+ * reference's EXACT mode at any batch size. Above 1024 picks out must be 16-byte aligned too and M*topk*max(H, I) <
+ * 2^29. That path uses the prefill workspace: gfl_register_layer reserves it for 1024 picks, gfl_grouped_reserve sizes it
+ * for more ahead of graph capture (otherwise the first call of a larger size grows it). */
 int gfl_moe_forward(gfl_ctx* ctx, int li, const uint16_t* x, const int64_t* sel, const void* w, int w_is_half, int M,
                     int topk, float* out, int mode, float act_limit, gfl_stream stream);
 
@@ -155,9 +156,9 @@ int gfl_moe_forward_noalloc(gfl_ctx* ctx, int li, const uint16_t* x, const int64
 
 /* mode: AUTO, AFFINE, EXACT or I16 (all computed bit-exact to EXACT), or MFMA. With MFMA the workgroups of a routed expert take up to 4 of its slots
  * per pass, so the expert's tiles are decoded once for all of them.
- * Environment: GFL_SLOTS_PER_PASS = 1, 2, 4 or 8 forces the number of (token, expert) slots one GEMV pass of
- * gfl_moe_forward accumulates (default: 1 up to M = 8, with a workgroup per slot; else 2, with a workgroup per expert
- * whose slots take passes; MFMA: min(M, 4)). Read once by gfl_ctx_create. */
+ * Environment: GFL_SLOTS_PER_PASS = 1, 2, 4 or 8 forces the number of (token, expert) slots one GEMV pass of the decode
+ * launches accumulates (default: 1 up to M = 8, with a workgroup per slot; else 2, with a workgroup per expert
+ * whose slots take passes; MFMA: min(M, 4)), and keeps calls of up to 1024 picks on them. Read once by gfl_ctx_create. */
 
 /* Routed-expert forward of one layer for prefill-sized M (the north star's MFMA grouped GEMM), same arguments and
  * result layout as gfl_moe_forward: x fp16 [M, H], sel int64 [M, topk] (ids outside [0, E) skipped), w fp16 or fp32

@@ -35,3 +35,45 @@ def test_chain_pass_sizes_bitexact(gpu, oracle, E, Ks):
     got = out.cpu().numpy()
     bad = {int(c): int(np.count_nonzero((got != want)[sel[:, 0] == e])) for e, c in zip(ids, COUNTS)}
     assert not any(bad.values()), {c: b for c, b in bad.items() if b}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,topk,E,skip,offset", [
+    (13, 5, 130, False, 0),     # 65 picks, half a pick per expert: the first call on the chains
+    (13, 5, 131, False, 0),     # just under half a pick per expert: the decode launches
+    (33, 2, 8, True, 0),        # few experts, picks skipped and out of range, a token without picks
+    (33, 2, 8, False, 4),       # an out that is not 16-byte aligned: the decode launches
+    (128, 8, 24, True, 0),      # 1,024 picks: the one-launch plan's largest call
+    (64, 16, 1024, False, 0),   # every expert id of the largest layer
+])
+def test_batched_decode_calls_bitexact(gpu, oracle, M, topk, E, skip, offset):
+    """Calls of 65..1,024 picks on either side of each line of the dispatch, against the oracle, bit for bit; three calls
+    in a row (the plan and workspace are reused)."""
+    import synth
+    import torch
+    from oracle import Mat
+    H, I, li, Ks = 512, 256, 65, (3, 3, 4)
+    L = synth.SynthLayer(li, E, H, I, Ks)
+    L.register(gpu, li)
+    rng = np.random.default_rng(M * 31 + E)
+    sel = np.stack([rng.choice(E, topk, replace=E < topk) for _ in range(M)]).astype(np.int64)
+    if skip:
+        r = rng.random(sel.shape)
+        sel[r < 0.2] = -1
+        sel[(r >= 0.2) & (r < 0.25)] = E + 7
+        sel[3] = -1
+    x16 = (rng.standard_normal((M, H)) * 0.4).astype(np.float16)
+    w = rng.random((M, topk)).astype(np.float16)
+    buf = torch.full((M * H + 4,), float("nan"), dtype=torch.float32, device="cuda")
+    out = buf[offset // 4:offset // 4 + M * H].view(M, H)
+    xd, sd, wd = torch.from_numpy(x16).cuda(), torch.from_numpy(sel).cuda(), torch.from_numpy(w).cuda()
+    need = sorted(int(e) for e in np.unique(sel) if 0 <= e < E)
+    mats = {e: tuple(Mat(*L.matrix(e, p), *((H, I) if p < 2 else (I, H)), Ks[p]) for p in range(3)) for e in need}
+    experts = [mats.get(e, mats[need[0]]) for e in range(E)]
+    want = oracle.moe_forward(experts, x16.astype(np.float32), np.where(sel < E, sel, -1), w.astype(np.float32), mode=1)
+    for k in range(3):
+        print(f"batched decode: M={M} topk={topk} E={E} skip={skip} offset={offset} call {k}", flush=True)
+        out.fill_(float("nan"))
+        gpu.moe_forward(li, xd, sd, wd, out)
+        torch.cuda.synchronize()
+        assert np.count_nonzero(out.cpu().numpy() != want) == 0
