@@ -102,10 +102,12 @@ __device__ __forceinline__ int gp_wave_scan(int v, int lane)
     return v;
 }
 
+constexpr int GP_HIST = 256;   // sizes the items' counting sort tells apart (4 per lane of a wave)
+
 // The GEMM's items: every expert's slots in passes of mt, a workgroup per pass (and column block), so that an expert
 // with many slots runs its passes side by side. Whole passes first, then the remainders by descending size: the longest
 // workgroups go first and the short ones fill the end of the launch. The remainders are placed by a counting sort over
-// their sizes (mt <= 127; ties in any order, the items are independent). Comparing every expert with every other
+// their sizes (mt <= GP_HIST; ties in any order, the items are independent). Comparing every expert with every other
 // instead took about 10 us of the plan at E = 288. Whole workgroup of GP_PLAN_THREADS, thread t = expert t: tot slots
 // from slot off; s_hist and s_full are LDS scratch; ends with a barrier.
 __device__ __forceinline__ void gp_items(int t, int E, int mt, int tot, int off, const GPlan& g, int* s_hist,
@@ -113,7 +115,7 @@ __device__ __forceinline__ void gp_items(int t, int E, int mt, int tot, int off,
 {
     const int lane = t & 63, wv = t >> 6;
     const int full = t < E ? tot / mt : 0, rem = t < E ? tot - full * mt : 0;
-    if (t < 128) s_hist[t] = 0;
+    if (t < GP_HIST) s_hist[t] = 0;
     const int finc = gp_wave_scan(full, lane);
     if (lane == 63) s_full[wv] = finc;
     __syncthreads();
@@ -128,10 +130,13 @@ __device__ __forceinline__ void gp_items(int t, int E, int mt, int tot, int off,
     __syncthreads();
     if (wv == 0)
     {
-        const int v0 = s_hist[127 - 2 * lane], v1 = s_hist[126 - 2 * lane];   // sizes descending over the lanes
-        const int inc = gp_wave_scan(v0 + v1, lane);
-        s_hist[127 - 2 * lane] = inc - v0 - v1;
-        s_hist[126 - 2 * lane] = inc - v1;
+        const int b = GP_HIST - 1 - 4 * lane;   // sizes descending over the lanes, four a lane
+        const int v0 = s_hist[b], v1 = s_hist[b - 1], v2 = s_hist[b - 2], v3 = s_hist[b - 3];
+        const int inc = gp_wave_scan(v0 + v1 + v2 + v3, lane);
+        s_hist[b] = inc - v0 - v1 - v2 - v3;
+        s_hist[b - 1] = inc - v1 - v2 - v3;
+        s_hist[b - 2] = inc - v2 - v3;
+        s_hist[b - 3] = inc - v3;
         if (lane == 63) g.hdr[2] = nfull + inc;
     }
     __syncthreads();
@@ -150,7 +155,7 @@ __global__ __launch_bounds__(GP_PLAN_THREADS) void gp_place_kernel(const int64_t
 {
     __shared__ int s_base[MAX_EXPERTS];
     __shared__ int s_off[MAX_EXPERTS];
-    __shared__ int s_hist[128];
+    __shared__ int s_hist[GP_HIST];
     __shared__ int s_wtot[GP_PLAN_WAVES], s_wjob[GP_PLAN_WAVES], s_wop[GP_PLAN_WAVES];
     __shared__ int s_bad;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
@@ -279,7 +284,7 @@ __global__ __launch_bounds__(GP_PLAN_THREADS) void gp_plan_kernel(const uint64_t
     __shared__ int s_off[MAX_EXPERTS];
     __shared__ int s_job[GP_PLAN_THREADS];    // job number of the slot, at the slots of job-opening picks
     __shared__ int s_pjob[GP_PLAN_THREADS];   // each pick's job, -1 if skipped
-    __shared__ int s_hist[128];
+    __shared__ int s_hist[GP_HIST];
     __shared__ int s_wtot[GP_PLAN_WAVES], s_wop[GP_PLAN_WAVES], s_full[GP_PLAN_WAVES];
     __shared__ int s_bad;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
@@ -789,6 +794,153 @@ __global__ __launch_bounds__(GP_NW * 64) void gp_gemm_kernel(GemmArgs a)
     }
 }
 
+// The same GEMM for experts with many slots: passes of up to GW_MT, so that a weight is decoded half as often. What bounds
+// it: the decode (72 VALU cycles per tile) and the MFMAs (8 per tile and 16 slots) share the SIMD's issue and overlap in
+// part. The accumulators take 80 VGPRs; the kernel fits 128 (4 waves per SIMD, two workgroups per CU) with groups of 4 tile
+// rows, whose input ring is 40 KB, and one input fragment in flight at a time. The input rows are swizzled instead of
+// padded: a load brings two rows, and their 128-byte chunks have to lie next to each other in LDS.
+// Measured against passes of 80 (ms per layer, E = 288 top-8, mean slots in brackets): M = 2048 [57] 1.60 -> 1.70, M = 2500
+// [69] 1.76 -> 1.80, M = 2700 [75] 2.00 -> 1.87, M = 4096 [114] 3.07 -> 2.42, M = 5000 [139] 3.43 -> 2.80, M = 8192 [228] 5.42 -> 4.86. Passes of 144:
+// 4096 2.41, 5000 3.02, 8192 4.80; of 176 (two registers spilled): 2.43, 2.80, 4.99.
+constexpr int GW_MT = 160;         // slots per pass (up to 10 MFMA row blocks)
+constexpr int GW_GR = 4;           // tile rows per group
+constexpr int GW_XPW = GW_MT / 2 / GP_NW;       // pairs of input rows each wave loads per group
+constexpr int GW_XROW = GW_GR * 16 * 2;         // input bytes of one slot per group
+
+template <int K>
+__global__ __launch_bounds__(GP_NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void gw_gemm_kernel(GemmArgs a)
+{
+    constexpr int TB = 32 * K, RB = GP_CPW * TB, GB = GW_GR * RB;
+    constexpr int NLD = GB / 256;                 // trellis dword loads per lane per group
+    static_assert(GB % 256 == 0 && GW_MT % (2 * GP_NW) == 0, "whole wave loads");
+    extern __shared__ __align__(16) uint8_t gp_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int nch = a.ndim / GP_WCOLS, per = nch * a.nmat;
+    const int xcd = blockIdx.x % 8, j = blockIdx.x / 8;
+    const int it = (j / per) * 8 + xcd, rr0 = j % per;
+    if (it >= a.nit || it >= a.g.hdr[2]) return;
+    const int4 item = a.g.item[it];
+    const int e = item.x, c0 = item.y, T = item.z;
+    const int nc = rr0 % nch;
+    const int mat = a.mat_base + rr0 / nch;
+    const int TN = a.ndim / 16, TK = a.kdim / 16, ngroups = TK / GW_GR;
+    const int t0 = (nc * GP_NW + wave) * GP_CPW;                     // this wave's first tile column
+    uint8_t* ring = gp_lds + wave * 2 * GB;                           // [2][GW_GR tile rows][GP_CPW columns][TB]
+    uint8_t* xring = gp_lds + GP_NW * 2 * GB;                         // [2][GW_MT slots][GW_XROW], swizzled
+    const uint8_t* tr = reinterpret_cast<const uint8_t*>(a.ptrs[(size_t)e * 9 + mat]);
+    const size_t gstride = (size_t)TN * TB;                           // bytes per tile row of the matrix
+    uint8_t* cb = const_cast<uint8_t*>(uniform_ptr(tr + (size_t)t0 * TB));
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(cb, (short)0, (int)((size_t)TK * gstride),
+                                                                        0x00020000);
+    const int gs = (int)gstride;
+    int voff[NLD];
+#pragma unroll
+    for (int i = 0; i < NLD; ++i)
+    {
+        const int byte = i * 256 + lane * 4;   // within the group's [GW_GR][GP_CPW][TB] block
+        voff[i] = (byte / RB) * gs + (byte % RB);
+    }
+    const LaneDec d = lane_dec(lane, K);
+    const uint16_t* xin = a.xin + (size_t)(mat - a.mat_base) * a.cap * a.kdim;
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(uniform_ptr(reinterpret_cast<const uint8_t*>(xin))), (short)0,
+        (int)((size_t)a.cap * a.kdim * 2), 0x00020000);
+    uint16_t* yout = a.yout + (size_t)(mat - a.mat_base) * a.cap * a.ndim;
+    const int q = lane >> 4, i16 = lane & 15;
+    // A load brings the group's chunks of two slots: lane l the 4 bytes at l % 32 of slot row l / 32. The chunk's
+    // 16-byte unit 2q + rp (rows 2rp, 2rp + 1 of lane group q) is at byte 64 q + 16 rp of the stored group of 8 tile
+    // rows; it lands at unit (2q + rp) ^ (pair % 8), so that the 16 rows of a fragment read lie in different banks.
+    const int un = (lane & 31) >> 2;
+    const int x1 = (un >> 1) * 64 + (un & 1) * 16 + (lane & 3) * 4;   // a pair whose second slot is past the pass repeats
+    const int x2 = x1 + (lane >> 5) * a.kdim * 2;                     // its first
+    auto issue = [&](int g) {
+        uint8_t* dst = ring + (g & 1) * GB;
+#pragma unroll
+        for (int i = 0; i < NLD; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (gp_lds_void*)(dst + i * 256), 4, voff[i], g * GW_GR * gs, 0, 0);
+        uint8_t* xd = xring + (g & 1) * GW_MT * GW_XROW;
+#pragma unroll
+        for (int k = 0; k < GW_XPW; ++k)
+        {
+            const int pr = wave + GP_NW * k;   // pair of slots, dealt over the waves
+            if (2 * pr < T)
+            {
+                const int sw = ((pr & 6) << 5) | ((pr & 1) << 4);   // unit pr % 8 as source bytes
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (gp_lds_void*)(xd + pr * 2 * GW_XROW), 4,
+                                                         (2 * pr + 1 < T ? x2 : x1) ^ sw,
+                                                         (c0 + 2 * pr) * a.kdim * 2 + (g >> 1) * 256 + (g & 1) * 32, 0, 0);
+            }
+        }
+    };
+    auto pass = [&](auto nmb_c) {
+        constexpr int NMB = decltype(nmb_c)::value;
+        float4v acc[GP_CPW][NMB];
+#pragma unroll
+        for (int c = 0; c < GP_CPW; ++c)
+#pragma unroll
+            for (int mb = 0; mb < NMB; ++mb) acc[c][mb] = float4v{ 0.f, 0.f, 0.f, 0.f };
+        // slot 16 mb + i16 is row i16 % 2 of pair 8 mb + i16 / 2
+        const int xr = i16 * GW_XROW + (((2 * q) ^ (i16 >> 1)) << 4);
+        issue(0);
+        for (int g = 0; g < ngroups; ++g)
+        {
+            gp_wait_vmcnt<0>();
+            gp_barrier();   // every wave's loads of group g landed; every wave is done with group g - 1
+            if (g + 1 < ngroups) issue(g + 1);
+            const uint8_t* sl = ring + (g & 1) * GB;
+            const uint8_t* xs = xring + (g & 1) * GW_MT * GW_XROW;
+#pragma unroll
+            for (int rp = 0; rp < GW_GR / 2; ++rp)
+            {
+                half8 B[GP_CPW];
+#pragma unroll
+                for (int c = 0; c < GP_CPW; ++c)
+                {
+                    const uint8_t* tp = sl + 2 * rp * RB + c * TB;
+                    const half4 B0 = decode4<K>(ld_u32(tp + d.o0), ld_u32(tp + d.o1), d.sh);
+                    const half4 B1 = decode4<K>(ld_u32(tp + RB + d.o0), ld_u32(tp + RB + d.o1), d.sh);
+                    B[c] = half8{ B0[0], B0[1], B0[2], B0[3], B1[0], B1[1], B1[2], B1[3] };
+                }
+                __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+                for (int mb = 0; mb < NMB; ++mb)
+                {
+                    const half8 A = *reinterpret_cast<const half8*>(xs + mb * 16 * GW_XROW + (xr ^ (rp << 4)));
+#pragma unroll
+                    for (int c = 0; c < GP_CPW; ++c)
+                        acc[c][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[c], acc[c][mb], 0, 0, 0);
+                }
+                __builtin_amdgcn_s_setprio(0);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < GP_CPW; ++c)
+#pragma unroll
+            for (int mb = 0; mb < NMB; ++mb)
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr)
+                {
+                    const int sl = mb * 16 + q * 4 + rr;
+                    if (sl < T)
+                        yout[(size_t)(c0 + sl) * a.ndim + (t0 + c) * 16 + i16] = (uint16_t)f2h_bits(acc[c][mb][rr]);
+                }
+    };
+    static_assert(GW_MT == 160, "one case per row-block count");
+    switch ((T + 15) / 16)
+    {
+        case 1: pass(std::integral_constant<int, 1>{}); break;
+        case 2: pass(std::integral_constant<int, 2>{}); break;
+        case 3: pass(std::integral_constant<int, 3>{}); break;
+        case 4: pass(std::integral_constant<int, 4>{}); break;
+        case 5: pass(std::integral_constant<int, 5>{}); break;
+        case 6: pass(std::integral_constant<int, 6>{}); break;
+        case 7: pass(std::integral_constant<int, 7>{}); break;
+        case 8: pass(std::integral_constant<int, 8>{}); break;
+        case 9: pass(std::integral_constant<int, 9>{}); break;
+        default: pass(std::integral_constant<int, 10>{}); break;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // EXACT for many slots: the reference's accumulator chains, each weight decoded once per pass of an expert's slots
 // ---------------------------------------------------------------------------------------------------------------
@@ -1083,14 +1235,38 @@ static int gp_gemm_launch(const GemmArgs& a, int nmat, hipStream_t st)
     return 0;
 }
 
-static int gp_gemm(int K, const GemmArgs& a, int nmat, hipStream_t st)
+template <int K>
+static int gw_gemm_launch(const GemmArgs& a, int nmat, hipStream_t st)
+{
+    constexpr size_t lds = (size_t)GP_NW * 2 * GW_GR * GP_CPW * 32 * K + (size_t)2 * GW_MT * GW_XROW;
+    static const bool opened = hipFuncSetAttribute(reinterpret_cast<const void*>(gw_gemm_kernel<K>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    if (!opened) return -1;
+    GemmArgs b = a;
+    b.nmat = nmat;
+    const unsigned grid = (unsigned)(((a.nit + 7) / 8) * 8 * (a.ndim / GP_WCOLS) * nmat);
+    hipLaunchKernelGGL(gw_gemm_kernel<K>, dim3(grid), dim3(GP_NW * 64), lds, st, b);
+    return 0;
+}
+
+// Slots per pass of an MFMA call of P picks over E experts: passes of GP_MT while an expert's mean share fits one with
+// room for its spread (measured at gw_gemm_kernel).
+static int gp_slots(int P, int E) { return P < 72 * E ? GP_MT : GW_MT; }
+
+template <int K>
+static int gp_gemm_k(int mt, const GemmArgs& a, int nmat, hipStream_t st)
+{
+    return mt == GW_MT ? gw_gemm_launch<K>(a, nmat, st) : gp_gemm_launch<K>(a, nmat, st);
+}
+
+static int gp_gemm(int K, int mt, const GemmArgs& a, int nmat, hipStream_t st)
 {
     switch (K)
     {
-        case 2: return gp_gemm_launch<2>(a, nmat, st);
-        case 3: return gp_gemm_launch<3>(a, nmat, st);
-        case 4: return gp_gemm_launch<4>(a, nmat, st);
-        case 5: return gp_gemm_launch<5>(a, nmat, st);
+        case 2: return gp_gemm_k<2>(mt, a, nmat, st);
+        case 3: return gp_gemm_k<3>(mt, a, nmat, st);
+        case 4: return gp_gemm_k<4>(mt, a, nmat, st);
+        case 5: return gp_gemm_k<5>(mt, a, nmat, st);
         default: return -1;
     }
 }
@@ -1193,32 +1369,33 @@ int launch_grouped(const uint64_t* ptrs, const int64_t* sel, const void* w, int 
                    hipStream_t st)
 {
     const int M = P / topk;
-    launch_grouped_plan(ptrs, sel, w, w_half, P, topk, E, GP_MT, g, st);
+    const int mt = gp_slots(P, E);
+    launch_grouped_plan(ptrs, sel, w, w_half, P, topk, E, mt, g, st);
     const int parts = prep_parts(P, H);
     hipLaunchKernelGGL(gp_prep_kernel<false>, dim3((unsigned)(((long)P * parts + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
                        ptrs, x, H, topk, cap, parts, g,
                        static_cast<void*>(xt));
     GemmArgs a;
-    a.ptrs = ptrs; a.kdim = H; a.ndim = I; a.cap = cap; a.nit = gemm_items(P, E, GP_MT); a.g = g; a.xin = xt; a.yout = ygu;
+    a.ptrs = ptrs; a.kdim = H; a.ndim = I; a.cap = cap; a.nit = gemm_items(P, E, mt); a.g = g; a.xin = xt; a.yout = ygu;
     if (Kg == Ku)
     {
         a.mat_base = 0;
-        if (gp_gemm(Kg, a, 2, st)) return -1;
+        if (gp_gemm(Kg, mt, a, 2, st)) return -1;
     }
     else
     {
         a.mat_base = 0;
-        if (gp_gemm(Kg, a, 1, st)) return -1;
+        if (gp_gemm(Kg, mt, a, 1, st)) return -1;
         GemmArgs b = a;
         b.mat_base = 1;
         b.xin = xt + (size_t)cap * H;
         b.yout = ygu + (size_t)cap * I;
-        if (gp_gemm(Ku, b, 1, st)) return -1;
+        if (gp_gemm(Ku, mt, b, 1, st)) return -1;
     }
     act_launch<false>(ptrs, P, I, cap, g, ygu, silu_tab, act_limit, xd, st);
     GemmArgs c = a;
     c.mat_base = 2; c.kdim = I; c.ndim = H; c.xin = xd; c.yout = yraw;
-    if (gp_gemm(Kd, c, 1, st)) return -1;
+    if (gp_gemm(Kd, mt, c, 1, st)) return -1;
     comb_launch(H, M, topk, g, yraw, out, st);
     return 0;
 }
