@@ -293,6 +293,42 @@ __device__ inline float fwht128_row(float (&v)[8])
     return (__builtin_popcount(L) & 1) ? -1.0f : 1.0f;
 }
 
+// Products with packed fp16 operands in one instruction each (v_fma_mix_f32 with -0 as the addend, which leaves every
+// product as it is, signed zeros included), instead of a conversion per operand and a multiply. Half h (0 low, 1 high) of
+// b, and of a where a is packed too: a product of two fp16 values is exact in fp32, one of an fp32 value is rounded once.
+// Measured: M = 2048 input transform 98.5 -> 95.8 us, combine 49.9 ->
+// 47.2 us; a layer of the single-token decode call (config 1) 43.4 -> 43.0 us.
+template <int H>
+__device__ __forceinline__ float mul_hh(uint32_t a, uint32_t b)
+{
+    float r;
+    const float nz = -0.0f;
+    if constexpr (H == 0) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(a), "v"(b), "s"(nz));
+    else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(r) : "v"(a), "v"(b), "s"(nz));
+    return r;
+}
+template <int H>
+__device__ __forceinline__ float mul_fh(float a, uint32_t b)
+{
+    float r;
+    const float nz = -0.0f;
+    if constexpr (H == 0) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[0,1,0]" : "=v"(r) : "v"(a), "v"(b), "s"(nz));
+    else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(a), "v"(b), "s"(nz));
+    return r;
+}
+
+// v[k] * the k-th of 8 packed fp16 scales
+__device__ __forceinline__ void mul8_fh(float (&v)[8], uint4 sc)
+{
+    const uint32_t sw[4] = { sc.x, sc.y, sc.z, sc.w };
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        v[2 * i] = mul_fh<0>(v[2 * i], sw[i]);
+        v[2 * i + 1] = mul_fh<1>(v[2 * i + 1], sw[i]);
+    }
+}
+
 __device__ __forceinline__ float h2f_lane(uint4 v, int k)
 {
     const uint32_t w = k < 2 ? v.x : k < 4 ? v.y : k < 6 ? v.z : v.w;
@@ -304,7 +340,10 @@ __device__ inline void out_block_row_rounded(float (&v)[8], uint4 sc)
 {
     const float sh = fwht128_row(v) * HADF;   // (sign * v) * HADF == v * (sign * HADF), bit for bit
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = r16(v[k] * sh * h2f_lane(sc, k));
+    for (int k = 0; k < 8; ++k) v[k] = v[k] * sh;
+    mul8_fh(v, sc);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = r16(v[k]);
 }
 
 // out_block (ft_core.h:105-110) on a 16-lane row: v = the lane's 8 fp32 outputs, sc its 8 fp16 scales
@@ -328,8 +367,7 @@ __device__ inline void out_block_row_h(float (&v)[8], uint4 raw, uint4 sc)
 // 8 fp16 scales; on return v = the fp32 products (H v) * HADF, each still to be rounded to fp16
 __device__ inline void prep_block_row_fp(float (&v)[8], uint4 sc)
 {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = v[k] * h2f_lane(sc, k);
+    mul8_fh(v, sc);
     const float sh = fwht128_row(v) * HADF;
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = v[k] * sh;
@@ -340,8 +378,11 @@ __device__ inline void prep_block_row_p(float (&v)[8], uint4 x, uint4 sc)
 {
     const uint32_t xw[4] = { x.x, x.y, x.z, x.w }, sw[4] = { sc.x, sc.y, sc.z, sc.w };
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-        v[k] = h2f_bits((uint16_t)(xw[k >> 1] >> (16 * (k & 1)))) * h2f_bits((uint16_t)(sw[k >> 1] >> (16 * (k & 1))));
+    for (int i = 0; i < 4; ++i)
+    {
+        v[2 * i] = mul_hh<0>(xw[i], sw[i]);
+        v[2 * i + 1] = mul_hh<1>(xw[i], sw[i]);
+    }
     const float sh = fwht128_row(v) * HADF;
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = v[k] * sh;

@@ -680,6 +680,15 @@ __device__ __forceinline__ float chain_relay(const uint8_t* __restrict__ col_bas
     // carries no branch around the status word's atomic
     bool waits_ok = true;
     const int nphp = (nph + PF - 1) / PF * PF;   // phases padded to whole rounds of PF (the padding has no work)
+    // With one wave per column the input transform runs before the loop instead of in its first phase, so that its
+    // registers are free in the loop: gate|up 128 -> 90, down 118 -> 96, 5 waves per SIMD instead of 4 (config 1, us per
+    // layer: M = 2 67.8 -> 66.5, M = 3 103.2 -> 96.8, M = 8 237.7 -> 235.4). With more waves per column, whose launches
+    // are sized to 3 waves per SIMD or fewer, the first-phase form is 1% faster.
+    if constexpr (RW == 1)
+    {
+        if (prio) __builtin_amdgcn_s_setprio(3);
+        pre();
+    }
     for (int ph0 = 0; ph0 < nphp; ph0 += PF)
     {
         // prio: the wave's issue priority falls from 3 to 0 over the quarters of its phases. A SIMD issues its
@@ -705,7 +714,8 @@ __device__ __forceinline__ float chain_relay(const uint8_t* __restrict__ col_bas
             // first trellis groups queue behind one another in HBM, and the inputs (x from L2, suh shared by the
             // expert's workgroups) land sooner, so the transform fills that wait (before the first group's decode it
             // measured 1.1 us faster at config 1 M=1 than after it)
-            if (ph == 0) pre();
+            if constexpr (RW > 1)
+                if (ph == 0) pre();
             // written in every phase, padding ones included (the slot is this wave's own and only its own decode
             // reads it): with the write under the phase's branch, the compiler's wait before it also covered the
             // younger of the groups in flight
@@ -1786,7 +1796,7 @@ static int resident_waves(const void* kern)
 // Progress priority of a relay launch (chain_relay's prio): on when the launch puts more than one wave on a SIMD and
 // all of them fit at once (cap: resident_waves), so that a SIMD's last wave would otherwise run its last stretch
 // alone. Measured on MI355X (config 1, us per token): M = 1 (gate|up 3 waves per SIMD of 3, down 2.5 of 4) 48.9 ->
-// 45.8; M = 2 with it on gate|up (3 of 4) 36.6 -> 34.9, while on down as well (5 waves per SIMD, two rounds) 0.4
+// 45.8; M = 2 with it on gate|up (3 of 4) 36.6 -> 34.9, while on a down launch of two rounds (5 waves per SIMD of 4) 0.4
 // slower; routed + shared expert in one call at M = 2 (gate|up 3.4 of 4) 42.4 -> 40.0. prio >= 0 (GFL_RELAY_PRIO)
 // forces it.
 static int relay_prio(int prio, long waves, int cap)
