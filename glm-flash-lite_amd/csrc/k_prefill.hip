@@ -889,29 +889,33 @@ __global__ __launch_bounds__(GP_NW * 64) __attribute__((amdgpu_waves_per_eu(4)))
             if (g + 1 < ngroups) issue(g + 1);
             const uint8_t* sl = ring + (g & 1) * GB;
             const uint8_t* xs = xring + (g & 1) * GW_MT * GW_XROW;
-#pragma unroll
-            for (int rp = 0; rp < GW_GR / 2; ++rp)
-            {
-                half8 B[GP_CPW];
+            half8 B[2][GP_CPW];
+            auto dec = [&](int rp, half8 (&o)[GP_CPW]) {
 #pragma unroll
                 for (int c = 0; c < GP_CPW; ++c)
                 {
                     const uint8_t* tp = sl + 2 * rp * RB + c * TB;
                     const half4 B0 = decode4<K>(ld_u32(tp + d.o0), ld_u32(tp + d.o1), d.sh);
                     const half4 B1 = decode4<K>(ld_u32(tp + RB + d.o0), ld_u32(tp + RB + d.o1), d.sh);
-                    B[c] = half8{ B0[0], B0[1], B0[2], B0[3], B1[0], B1[1], B1[2], B1[3] };
+                    o[c] = half8{ B0[0], B0[1], B0[2], B0[3], B1[0], B1[1], B1[2], B1[3] };
                 }
-                __builtin_amdgcn_s_setprio(1);
+            };
+            // the whole group's decode first, then its MFMAs in one run (decode and MFMAs of each row pair in turn: M = 4096
+            // 2.38 ms against 2.31)
+            dec(0, B[0]);
+            dec(1, B[1]);
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int rp = 0; rp < GW_GR / 2; ++rp)
 #pragma unroll
                 for (int mb = 0; mb < NMB; ++mb)
                 {
                     const half8 A = *reinterpret_cast<const half8*>(xs + mb * 16 * GW_XROW + (xr ^ (rp << 4)));
 #pragma unroll
                     for (int c = 0; c < GP_CPW; ++c)
-                        acc[c][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[c], acc[c][mb], 0, 0, 0);
+                        acc[c][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[rp][c], acc[c][mb], 0, 0, 0);
                 }
-                __builtin_amdgcn_s_setprio(0);
-            }
+            __builtin_amdgcn_s_setprio(0);
         }
 #pragma unroll
         for (int c = 0; c < GP_CPW; ++c)
