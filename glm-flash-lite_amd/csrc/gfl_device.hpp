@@ -205,13 +205,30 @@ __device__ inline int gp_perm_pos(int b, int r)
     return b * 128 + q * 32 + tr * 4 + jj;
 }
 
-// Elements 8li..8li+7 of block b in the GEMM input layout gp_perm_pos: pairs (2q, 2q + 1) are adjacent, at
-// b * 128 + q * 32 + (li >> 1) * 4 + 2 * (li & 1)
+// Exchange between lane pairs L, L ^ W inside quads (W = 1 or 2): afterwards the lower lane of a pair holds both lanes'
+// x, the upper one both lanes' y.
+template <int W>
+__device__ __forceinline__ void quad_swap(uint32_t& x, uint32_t& y, bool upper)
+{
+    constexpr int CTRL = W == 1 ? 0xB1 : 0x4E;
+    const uint32_t px = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true);
+    const uint32_t py = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)y, CTRL, 0xF, 0xF, true);
+    x = upper ? py : x;
+    y = upper ? y : px;
+}
+
+// Elements 8li..8li+7 of block b in the GEMM input layout gp_perm_pos: pairs (2q, 2q + 1) = o[q] are adjacent, at
+// b * 128 + q * 32 + 2 li. A 4x4 transposition inside each quad of lanes gives lane li the pairs of lanes li & ~3 .. li | 3
+// for q = li % 4, 16 contiguous bytes: one store instead of four of 4 bytes (the grouped path's input transform at M = 8192,
+// which writes 1.34 GB: 453 -> 420 us).
 __device__ __forceinline__ void gp_store_row(uint16_t* dst, int b, int li, const uint32_t (&o)[4])
 {
-    uint16_t* d0 = dst + b * 128 + (li >> 1) * 4 + 2 * (li & 1);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t*>(d0 + q * 32) = o[q];
+    uint32_t t0 = o[0], t1 = o[1], t2 = o[2], t3 = o[3];
+    quad_swap<1>(t0, t1, li & 1);
+    quad_swap<1>(t2, t3, li & 1);
+    quad_swap<2>(t0, t2, li & 2);
+    quad_swap<2>(t1, t3, li & 2);
+    *reinterpret_cast<uint4*>(dst + b * 128 + (li & 3) * 32 + (li >> 2) * 8) = make_uint4(t0, t1, t2, t3);
 }
 
 __device__ inline float h2f_bits(uint16_t h) { __half x; __builtin_memcpy(&x, &h, 2); return __half2float(x); }
