@@ -644,12 +644,15 @@ static int run_chains(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64
 
 // Whether an EXACT call takes the accumulator-chain GEMMs on the grouped plan (run_chains) instead of the decode
 // launches: always above MAX_PICKS picks; below, from half a pick per expert on, three quarters where gate and up have
-// different bits and so a launch each (and above the 64 picks of the relay launches). The chain GEMM decodes an expert's weights once for all its slots, the decode launches once per 2 slots,
-// but it takes six launches instead of three. Measured (decode launches -> chains, us per layer, top-8; picks per expert in
-// brackets): E = 288, uniform routing: M = 9 [0.25] 261 -> 260, M = 16 [0.44] 420 -> 413, M = 24 [0.67] 600 -> 553, M = 64
-// [1.8] 1353 -> 1055; gate 3 and up 5 bits M = 18 [0.5] 515 -> 530, M = 27 [0.75] 705 -> 658; H=2048 I=768 M = 9 75 -> 82,
-// M = 16 117 -> 117, M = 24 153 -> 142, gate 3 up 5 bits M = 22 157 -> 165, M = 27 181 -> 177; E = 72: M = 9 [1] 259 -> 240, M = 64 [7.1] 1250 -> 526; Zipf 1.1 over 288: M = 16
-// 527 -> 329, M = 32 991 -> 445.
+// different bits and so a launch each (and above the 64 picks of the relay launches). The chain GEMM decodes an expert's
+// weights once per pass of 16 to 64 slots, the decode launches once per 2 slots, but it takes six launches instead of three.
+// Measured (decode launches -> chains, us per layer, top-8; picks per expert in brackets):
+//   E = 288, uniform routing: M = 9 [0.25] 261 -> 260, M = 16 [0.44] 420 -> 413, M = 24 [0.67] 600 -> 553,
+//     M = 64 [1.8] 1353 -> 1055; Zipf 1.1: M = 16 527 -> 329, M = 32 991 -> 445
+//   gate 3 and up 5 bits: M = 18 [0.5] 515 -> 530, M = 27 [0.75] 705 -> 658
+//   H = 2048, I = 768: M = 9 75 -> 82, M = 16 117 -> 117, M = 24 153 -> 142; gate 3 and up 5 bits M = 22 157 -> 165,
+//     M = 27 181 -> 177
+//   E = 72: M = 9 [1] 259 -> 240, M = 64 [7.1] 1250 -> 526
 // The chains' combine writes 16 bytes at a time, and the forced launch shapes (GFL_SLOTS_PER_PASS, GFL_RELAY) name the
 // decode launches, so an unaligned out and a context with either keep those.
 static bool takes_chains(const gfl_ctx* c, const Layer& L, int P, int mode, const float* out)

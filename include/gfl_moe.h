@@ -111,8 +111,8 @@ int gfl_layer_info(gfl_ctx* ctx, int li, int* info);
  * Empty calls, as the reference's tier_forward takes them (ft_tier_ext.cpp:893-903): M = 0 does nothing (every
  * buffer may be NULL); topk = 0 writes M rows of zeros to out (sel and w may be NULL).
  * M*topk <= 64, and up to 1024 with fewer than half a pick per expert of the layer (three quarters where gate and up
- * have different bits), mode MFMA or an out that is not 16-byte aligned: the decode launches. Other calls up to M*topk = 65536 (EXACT modes only; MFMA is refused above 1024):
- * the grouped plan of the prefill path, then the reference's accumulator chains (each chain step one element of a K=1
+ * have different bits), mode MFMA or an out that is not 16-byte aligned: the decode launches. Other calls up to
+ * M*topk = 65536 (EXACT modes only; MFMA is refused above 1024): the grouped plan of the prefill path, then the reference's accumulator chains (each chain step one element of a K=1
  * fp32 MFMA, i.e. an fmaf), each weight decoded once per pass of up to 64 of an expert's slots, bit-identical to the
  * reference's EXACT mode at any batch size. Above 1024 picks out must be 16-byte aligned too and M*topk*max(H, I) <
  * 2^29. That path uses the prefill workspace: gfl_register_layer reserves it for 1024 picks, gfl_grouped_reserve sizes it
