@@ -556,6 +556,94 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_act_kernel(const uint64_t* __re
     }
 }
 
+// The same for calls of many picks, with the middle of the silu table in LDS. Each gate element is a lookup at an address
+// of its own, which from L1 takes the kernel a cycle per lane: at M = 8192 (top-8, I = 1536) about 160 of its 274 us. A
+// workgroup of 16 waves fills a CU's registers, holds the binades [2^-12, 16) of both signs (128 KB; other gates read
+// the table in memory) and goes through the (slot, 12 blocks) items, consecutive ones side by side, so that the fill is
+// paid once per CU. At M = 8192 it moves its 604 MB at 3.1 TB/s (before 2.2). Measured, gp_act_kernel -> this one, us, MFMA grouped
+// inputs | fp32 chain inputs, E = 288: M = 250 12.2 -> 15.6 | 12.7 -> 15.1, M = 512 19.4 -> 17.8 | 20.6 -> 18.1, M = 768
+// 27.2 -> 27.9 | 29.6 -> 27.9, M = 1024 34.7 -> 30.3 | 39.4 -> 29.9, M = 2048 71.0 -> 56.9 | 74.6 -> 51.0, M = 8192 274 ->
+// 196 | 299 -> 185: taken from 8,192 picks on, where every wave has at least two items at I = 1536.
+constexpr int GL_NW = 16;          // waves per workgroup
+constexpr int GL_CUS = 256;        // workgroups: one per CU
+constexpr int GL_MIN = 8192;       // picks from which the launch is taken
+constexpr int GL_LO = 3 << 10;     // first fp16 pattern held (2^-12), and how many of each sign
+constexpr int GL_N = 16 << 10;
+
+template <bool XL>
+__global__ __launch_bounds__(GL_NW * 64) void gl_act_kernel(const uint64_t* __restrict__ ptrs, int I, int cap, GPlan g,
+                                                            const uint16_t* __restrict__ ygu,
+                                                            const float* __restrict__ silu_tab, float act_limit,
+                                                            void* __restrict__ xd_out)
+{
+    __shared__ __align__(16) float tab[2 * GL_N];
+    for (int i = threadIdx.x; i < 2 * GL_N / 4; i += GL_NW * 64)
+        reinterpret_cast<float4*>(tab)[i] =
+            reinterpret_cast<const float4*>(silu_tab + GL_LO + (i < GL_N / 4 ? 0 : 0x8000 - GL_N))[i];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, rl = lane >> 4, li = lane & 15;
+    const int nbi = I / 128, nch = (nbi + 4 * GP_TA - 1) / (4 * GP_TA), items = g.hdr[0] * nch;
+    for (int item = blockIdx.x * GL_NW + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); item < items;
+         item += gridDim.x * GL_NW)
+    {
+        const int s = item / nch, c0 = (item % nch) * 4 * GP_TA;
+        const uint64_t* pe = ptrs + (size_t)g.slot_e[s] * 9;
+        const gptr<uint16_t> svh_g = gaddr<uint16_t>(pe[4]);
+        const gptr<uint16_t> svh_u = gaddr<uint16_t>(pe[6]);
+        const gptr<uint16_t> suh_d = gaddr<uint16_t>(pe[7]);
+        const uint16_t* yg = ygu + (size_t)s * I;
+        const uint16_t* yu = ygu + ((size_t)cap + s) * I;
+        uint4 gh[GP_TA], uh[GP_TA], sg[GP_TA], su[GP_TA], sd[GP_TA];
+#pragma unroll
+        for (int k = 0; k < GP_TA; ++k)
+        {
+            const int o = min(c0 + 4 * k + rl, nbi - 1) * 128 + li * 8;
+            gh[k] = *reinterpret_cast<const uint4*>(yg + o);
+            uh[k] = *reinterpret_cast<const uint4*>(yu + o);
+            sg[k] = gld16(svh_g, o);
+            su[k] = gld16(svh_u, o);
+            sd[k] = gld16(suh_d, o);
+        }
+        __builtin_amdgcn_sched_barrier(0);   // every load goes out before the first is used
+#pragma unroll
+        for (int k = 0; k < GP_TA; ++k)
+        {
+            float gv[8], uv[8];
+            out_block_row_h(gv, gh[k], sg[k]);
+            uint32_t gb[8], far = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+            {
+                gb[j] = f2h_bits(gv[j]) & 0xFFFFu;
+                const uint32_t m = (gb[j] & 0x7FFFu) - (uint32_t)GL_LO;
+                far = max(far, m);
+                gv[j] = tab[min(m, (uint32_t)GL_N - 1) + (gb[j] >> 15) * GL_N];
+            }
+            if (far >= (uint32_t)GL_N)
+            {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if ((gb[j] & 0x7FFFu) - (uint32_t)GL_LO >= (uint32_t)GL_N) gv[j] = silu_tab[gb[j]];
+            }
+            out_block_row_h(uv, uh[k], su[k]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) gv[j] = r16(act_mul_s(gv[j], uv[j], act_limit));
+            const int b = c0 + 4 * k + rl;
+            if constexpr (XL)
+            {
+                prep_block_row_fp(gv, sd[k]);
+                if (b < nbi) xg_store_row(static_cast<float*>(xd_out) + (size_t)s * I, b, li, gv);
+            }
+            else
+            {
+                uint32_t ah[4];
+                prep_block_row_fh(ah, gv, sd[k]);
+                if (b < nbi) gp_store_row(static_cast<uint16_t*>(xd_out) + (size_t)s * I, b, li, ah);
+            }
+        }
+    }
+}
+
 // out_block (ft_core.h:1016) of every expert output block and the weighted sum in job order (ft_core.h:1020-1033),
 // one wave per (token, group of 4 blocks): each 16-lane row takes one block; lane k < npk holds the token's k-th pick
 // (slot, weight, output scales), read back per pick with readlane; eight picks' loads are issued before their eight
@@ -1367,7 +1455,10 @@ static void act_launch(const uint64_t* ptrs, int P, int I, int cap, const GPlan&
                        const float* silu_tab, float act_limit, void* xd, hipStream_t st)
 {
     if (P <= GP_SMALL) act_launch_ta<XL, 1>(ptrs, P, I, cap, g, ygu, silu_tab, act_limit, xd, st);
-    else act_launch_ta<XL, GP_TA>(ptrs, P, I, cap, g, ygu, silu_tab, act_limit, xd, st);
+    else if (P < GL_MIN) act_launch_ta<XL, GP_TA>(ptrs, P, I, cap, g, ygu, silu_tab, act_limit, xd, st);
+    else
+        hipLaunchKernelGGL(gl_act_kernel<XL>, dim3(GL_CUS), dim3(GL_NW * 64), 0, st, ptrs, I, cap, g, ygu, silu_tab,
+                           act_limit, xd);
 }
 
 static void comb_launch(int H, int M, int topk, const GPlan& g, const uint16_t* yraw, float* out, hipStream_t st)
