@@ -221,6 +221,7 @@ __device__ __forceinline__ void quad_swap(uint32_t& x, uint32_t& y, bool upper)
 // b * 128 + q * 32 + 2 li. A 4x4 transposition inside each quad of lanes gives lane li the pairs of lanes li & ~3 .. li | 3
 // for q = li % 4, 16 contiguous bytes: one store instead of four of 4 bytes (the grouped path's input transform at M = 8192,
 // which writes 1.34 GB: 453 -> 420 us).
+template <bool NT = false>
 __device__ __forceinline__ void gp_store_row(uint16_t* dst, int b, int li, const uint32_t (&o)[4])
 {
     uint32_t t0 = o[0], t1 = o[1], t2 = o[2], t3 = o[3];
@@ -228,7 +229,10 @@ __device__ __forceinline__ void gp_store_row(uint16_t* dst, int b, int li, const
     quad_swap<1>(t2, t3, li & 1);
     quad_swap<2>(t0, t2, li & 2);
     quad_swap<2>(t1, t3, li & 2);
-    *reinterpret_cast<uint4*>(dst + b * 128 + (li & 3) * 32 + (li >> 2) * 8) = make_uint4(t0, t1, t2, t3);
+    typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+    uint4v* d = reinterpret_cast<uint4v*>(dst + b * 128 + (li & 3) * 32 + (li >> 2) * 8);
+    if constexpr (NT) __builtin_nontemporal_store(uint4v{ t0, t1, t2, t3 }, d);
+    else *d = uint4v{ t0, t1, t2, t3 };
 }
 
 __device__ inline float h2f_bits(uint16_t h) { __half x; __builtin_memcpy(&x, &h, 2); return __half2float(x); }

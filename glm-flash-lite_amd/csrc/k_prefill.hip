@@ -410,8 +410,9 @@ __device__ __forceinline__ void xg_store_row(float* dst, int b, int li, const fl
 }
 
 // prep_block (ft_core.h:97-102) of the gate and up inputs of slot s, `parts` waves per slot (prep_parts). XL: fp32 in the
-// accumulator-chain layout (xg_store_row), else fp16 in the MFMA layout (gp_store_row).
-template <bool XL>
+// accumulator-chain layout (xg_store_row), else fp16 in the MFMA layout (gp_store_row), NT:
+// with non-temporal stores.
+template <bool XL, bool NT>
 __global__ __launch_bounds__(GP_TW * 64) void gp_prep_kernel(const uint64_t* __restrict__ ptrs,
                                                              const uint16_t* __restrict__ x, int H, int topk, int cap,
                                                              int parts, GPlan g, void* __restrict__ xt_out)
@@ -468,8 +469,8 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_prep_kernel(const uint64_t* __r
                 prep_block_row_h(v, xv[buf][k], g1[buf][k]);
                 if (b < nblk)
                 {
-                    gp_store_row(d0, b, li, u);
-                    gp_store_row(d1, b, li, v);
+                    gp_store_row<NT>(d0, b, li, u);
+                    gp_store_row<NT>(d1, b, li, v);
                 }
             }
         }
@@ -1477,7 +1478,11 @@ int launch_grouped(const uint64_t* ptrs, const int64_t* sel, const void* w, int 
     const int mt = gp_slots(P, E);
     launch_grouped_plan(ptrs, sel, w, w_half, P, topk, E, mt, g, st);
     const int parts = prep_parts(P, H);
-    hipLaunchKernelGGL(gp_prep_kernel<false>, dim3((unsigned)(((long)P * parts + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
+    // inputs of 512 MB and more, which no cache keeps until the GEMM reads them, are stored non-temporally: H = 4096, M = 8192
+    // (1.07 GB) 318 -> 261 us, whole call at H = 5120 4478 -> 4386; of 134 MB 39.4 -> 37.4, of 268 MB 72.0 -> 73.1, whole call
+    // of 2,048 tokens at H = 5120 1582 -> 1584
+    const auto prep = (long)P * H < (1L << 27) ? gp_prep_kernel<false, false> : gp_prep_kernel<false, true>;
+    hipLaunchKernelGGL(prep, dim3((unsigned)(((long)P * parts + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
                        ptrs, x, H, topk, cap, parts, g,
                        static_cast<void*>(xt));
     GemmArgs a;
@@ -1514,7 +1519,7 @@ int launch_chains_gate_up(const uint64_t* ptrs, const int64_t* sel, const void* 
     const int ms = xg_slots(P, E);
     launch_grouped_plan(ptrs, sel, w, w_half, P, topk, E, ms, g, st);
     const int parts = prep_parts(P, H);
-    hipLaunchKernelGGL(gp_prep_kernel<true>, dim3((unsigned)(((long)P * parts + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
+    hipLaunchKernelGGL((gp_prep_kernel<true, false>), dim3((unsigned)(((long)P * parts + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
                        ptrs, x, H, topk, cap, parts, g, static_cast<void*>(xt));
     XgArgs a;
     a.ptrs = ptrs; a.kdim = H; a.ndim = I; a.cap = cap; a.nit = gemm_items(P, E, ms); a.g = g; a.xin = xt; a.yout = ygu;

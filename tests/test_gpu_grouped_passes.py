@@ -31,3 +31,27 @@ def test_wide_and_narrow_passes_are_equal(gpu, H, I, Ks):
     assert torch.equal(wide, narrow)
     d, rms = (wide - exact).double(), exact.double().square().mean().sqrt()
     assert float(d.square().mean().sqrt() / rms) <= 1e-3 and float(d.abs().max() / rms) <= 1e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [32767, 32768, 32771])
+def test_non_temporal_inputs(gpu, M):
+    """The input transform's stores around the size from which they are non-temporal (2^27 elements): one call equals
+    calls below it bit for bit (one pick per token, so no sum's order depends on the rest of the call)."""
+    import synth
+    import torch
+    H = 4096
+    L = synth.SynthLayer(74, 6, H, 256, (3, 3, 3))
+    L.register(gpu, 74)
+    gen = torch.Generator("cuda").manual_seed(M)
+    x = (torch.randn((M, H), generator=gen, device="cuda") * 0.4).half()
+    s = torch.randint(0, 6, (M, 1), generator=gen, device="cuda")
+    w = torch.rand((M, 1), generator=gen, device="cuda")
+    one, parts = (torch.full((M, H), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2))
+    print(f"non-temporal inputs: M={M}", flush=True)
+    gpu.grouped_forward(74, x, s, w, one)
+    for a in range(0, M, 12000):
+        b = min(a + 12000, M)
+        gpu.grouped_forward(74, x[a:b], s[a:b], w[a:b], parts[a:b])
+    torch.cuda.synchronize()
+    assert torch.equal(one, parts)
