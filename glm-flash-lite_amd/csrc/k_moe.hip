@@ -681,12 +681,23 @@ __device__ __forceinline__ float chain_relay(const uint8_t* __restrict__ col_bas
     bool waits_ok = true;
     const int nphp = (nph + PF - 1) / PF * PF;   // phases padded to whole rounds of PF (the padding has no work)
     // With one wave per column the input transform runs before the loop instead of in its first phase, so that its
-    // registers are free in the loop: gate|up 128 -> 90, down 118 -> 96, 5 waves per SIMD instead of 4 (config 1, us per
-    // layer: M = 2 67.8 -> 66.5, M = 3 103.2 -> 96.8, M = 8 237.7 -> 235.4). With more waves per column, whose launches
-    // are sized to 3 waves per SIMD or fewer, the first-phase form is 1% faster.
+    // registers are free in the loop, and the loop reads the inputs four tiles at a time: gate|up 128 -> 76 VGPRs, down
+    // 118 -> 80 (K = 5: 144 -> 92 and 134 -> 96), 6 waves per SIMD instead of 4 (K = 5: 5 instead of 3). At M = 4
+    // (config 1) gate|up puts 6 waves on a SIMD: with 4 resident they run as 4 + 2, with 5 (all 8 tiles' inputs read at
+    // once, 92 VGPRs) as 5 + 1, where the last wave runs alone, with 6 in one round. The decode's per-lane constants are
+    // made opaque to the compiler before the transform, which hides them under the inputs' latency: sunk below its barrier
+    // they cost every wave of a short launch 75 instructions (H = 1024, M = 4: 0.6 us). us per layer, transform in the
+    // first phase -> before the loop with 5 waves -> this form, runs of the three interleaved: config 1 M = 2 66.6 -> 64.5
+    // -> 63.3, M = 3 102.5 -> 94.8 -> 93.5, M = 4 126.8 -> 124.8 -> 114.1, M = 8 240.8 -> 236.3 -> 228.6; 4/4/3 bits, Zipf
+    // 1.1, M = 4 124.3 -> 124.4 -> 113.9 (on a slower card 129.8 -> 132.0 with 5 waves); H = 2048, I = 768, M = 4 34.4 ->
+    // 34.7 -> 34.1; H = 1024, I = 512, M = 4 20.3 -> 21.1 -> 20.5. With more waves per column, whose launches are sized to
+    // 3 waves per SIMD or fewer, the first-phase form is 1% faster.
     if constexpr (RW == 1)
     {
         if (prio) __builtin_amdgcn_s_setprio(3);
+        uint2 pm;
+        __builtin_memcpy(&pm, &Pm, 8);
+        asm volatile("" ::"v"(d.o0), "v"(d.o1), "v"(d.sh), "v"(pm.x), "v"(pm.y));
         pre();
     }
     for (int ph0 = 0; ph0 < nphp; ph0 += PF)
@@ -697,10 +708,9 @@ __device__ __forceinline__ float chain_relay(const uint8_t* __restrict__ col_bas
         // those behind, so the waves of a SIMD end together.
         if (prio)
         {
-            const int q4 = (4 * ph0) / nphp;
-            if (q4 == 0) __builtin_amdgcn_s_setprio(3);
-            else if (q4 == 1) __builtin_amdgcn_s_setprio(2);
-            else if (q4 == 2) __builtin_amdgcn_s_setprio(1);
+            if (4 * ph0 < nphp) __builtin_amdgcn_s_setprio(3);
+            else if (2 * ph0 < nphp) __builtin_amdgcn_s_setprio(2);
+            else if (4 * ph0 < 3 * nphp) __builtin_amdgcn_s_setprio(1);
             else __builtin_amdgcn_s_setprio(0);
         }
 #pragma unroll
@@ -734,7 +744,7 @@ __device__ __forceinline__ float chain_relay(const uint8_t* __restrict__ col_bas
                     cw[rr] = __builtin_amdgcn_mfma_f32_16x16x16f16(Pm, decode4<K>(hi, lo, d.sh), zero, 0, 0, 0);
                 }
             }
-            if (mine)
+            if (RW > 1 && mine)
             {
 #pragma unroll
                 for (int rr = 0; rr < 8; ++rr)
@@ -753,6 +763,14 @@ __device__ __forceinline__ float chain_relay(const uint8_t* __restrict__ col_bas
 #pragma unroll
                 for (int rr = 0; rr < 8; ++rr)
                 {
+                    if (RW == 1 && rr % 4 == 0)
+                    {
+                        // four tiles' inputs at a time (left to itself the compiler reads all eight before the FMAs)
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int i = rr; i < rr + 4; ++i)
+                            xf[i] = *reinterpret_cast<const float4v*>(lds_x + ((size_t)g * 8 + i) * 16 + j * 4);
+                    }
                     acc = __builtin_fmaf(cw[rr][0], xf[rr][0], acc);
                     acc = __builtin_fmaf(cw[rr][1], xf[rr][1], acc);
                     acc = __builtin_fmaf(cw[rr][2], xf[rr][2], acc);
@@ -1392,7 +1410,8 @@ __host__ __device__ constexpr size_t gu_relay_lds(int H, int P, int E)
 // order itself).
 // The last of the workgroups covering a 128-block of a pick (gate and up) runs its SwiGLU stage, as in gu_kernel.
 template <int K, int RW>
-__global__ __launch_bounds__(GU_NW * 64) __attribute__((amdgpu_waves_per_eu(3))) void gu_relay_kernel(GuArgs a)
+__global__ __launch_bounds__(GU_NW * 64) __attribute__((amdgpu_waves_per_eu(RW > 1 ? 3 : K == 5 ? 5 : 6))) void
+gu_relay_kernel(GuArgs a)
 {
     constexpr int NW = GU_NW, CW = NW / RW, TB = 32 * K;
     static_assert(NW % RW == 0, "relay width divides the workgroup");
@@ -1520,7 +1539,8 @@ __host__ __device__ constexpr size_t dn_relay_lds(int I)
 // job order it forms itself from sel (relay_combine_list; wave 0 loads the call's picks, weights and svh_down
 // addresses into registers before the GEMV, so none of their latency falls on that tail).
 template <int K, int RW>
-__global__ __launch_bounds__(GU_NW * 64) __attribute__((amdgpu_waves_per_eu(3))) void dn_relay_kernel(DnArgs a)
+__global__ __launch_bounds__(GU_NW * 64) __attribute__((amdgpu_waves_per_eu(RW > 1 ? 3 : 5))) void
+dn_relay_kernel(DnArgs a)
 {
     constexpr int NW = GU_NW, CW = NW / RW, TB = 32 * K, NQ = 128 / (16 * CW);
     extern __shared__ __align__(16) uint8_t lds_raw[];
