@@ -1101,17 +1101,20 @@ struct XgArgs
 // Input rows are swizzled by the loads' source addresses: the 16-byte unit u of slot m's row chunk lands at unit
 // u ^ (m % 8), so that the 16 slots a fragment read takes at one unit lie in different banks (row stride 512 bytes).
 // Occupancy: the accumulators take MS VGPRs, so 16-, 32- and 64-slot passes fit 64, 80 and 128 registers (8, 6 and 4
-// waves per SIMD, 4, 3 and 2 workgroups per CU; their LDS fits too). With few slots the loop lives from other waves'
-// issue slots: M = 64 decode call, 16-slot passes at 6 and 8 waves 1087 and 1073 us, 32-slot ones at 4 and 6 waves 1263
-// and 1098 us.
+// waves per SIMD, 4, 3 and 2 workgroups per CU), with nothing spilled as long as the trellis loads' addresses are scalar: a
+// register per load left seven of the twelve instantiations 2 to 5 short, reloaded inside the loops at K = 4 and 5 (4/4/4
+// bits, M = 64 1148 -> 1108 us, M = 128 1558 -> 1499, M = 333 2300 -> 2216; 3 bits M = 333 2186 -> 2151, others equal). LDS:
+// 4 K + MS KB a workgroup, so all of these fit but K = 5 at 64 slots, which has one workgroup per CU (xg_slots). With few
+// slots the loop lives from other waves' issue slots: M = 64 decode call, 16-slot passes at 6 and 8 waves 1087 and 1073 us,
+// 32-slot ones at 4 and 6 waves 1263 and 1098 us.
 template <int K, int MS>
 __global__ __launch_bounds__(XG_NW * 64) __attribute__((amdgpu_waves_per_eu(MS >= 64 ? 4 : MS >= 32 ? 6 : 8))) void
 xg_gemm_kernel(XgArgs a)
 {
     constexpr int TB = 32 * K, RB = XG_TC * TB, GB = 8 * RB, NG = XG_NG, XGB = MS * XG_XROW;
-    constexpr int NLD = GB / 256 / XG_NW;      // trellis dword loads per lane per group (the waves share a group)
+    constexpr int NLD = RB / 256;              // trellis dword loads per lane per group: wave r brings tile row r
     constexpr int RPW = MS / XG_NW;            // input rows each wave loads per group
-    static_assert(GB % (256 * XG_NW) == 0, "a group of tiles splits into whole loads of the waves");
+    static_assert(XG_NW == 8 && RB % 256 == 0, "a tile row of the group is whole loads of one wave");
     extern __shared__ __align__(16) uint8_t xg_lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nch = a.ndim / XG_COLS, per = nch * a.nmat;
@@ -1130,13 +1133,6 @@ xg_gemm_kernel(XgArgs a)
     uint8_t* cb = const_cast<uint8_t*>(uniform_ptr(tr + (size_t)nc * XG_TC * TB));
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(cb, (short)0, (int)((size_t)TK * gs),
                                                                         0x00020000);
-    int voff[NLD];
-#pragma unroll
-    for (int i = 0; i < NLD; ++i)
-    {
-        const int byte = (wave * NLD + i) * 256 + lane * 4;   // within the group's [8][XG_TC][TB] block
-        voff[i] = (byte / RB) * gs + (byte % RB);
-    }
     const float* xin = a.xin + (size_t)(mat - a.mat_base) * a.cap * a.kdim;
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t*>(uniform_ptr(reinterpret_cast<const uint8_t*>(xin))), (short)0,
@@ -1158,8 +1154,8 @@ xg_gemm_kernel(XgArgs a)
         uint8_t* dst = tring + (g % NG) * GB;
 #pragma unroll
         for (int i = 0; i < NLD; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (gp_lds_void*)(dst + (wave * NLD + i) * 256), 4, voff[i],
-                                                     g * 8 * gs, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (gp_lds_void*)(dst + (wave * NLD + i) * 256), 4, lane * 4,
+                                                     (g * 8 + wave) * gs + i * 256, 0, 0);
         // this wave's RPW slot rows of the group (rows of slots past the pass repeat its last slot); the lane's source
         // unit is permuted so that the row's 16-byte units land swizzled
         uint8_t* xd = xring + (g % NG) * XGB;

@@ -53,3 +53,11 @@ def test_one_wave_relay_launches_fit_their_waves(kernels, K):
     for name in ("gu_relay_kernel", "dn_relay_kernel"):
         k = kernels["%s<%d, 1>" % (name, K)]
         assert _waves(k) >= (5 if K == 5 else 6) and k[".vgpr_spill_count"] == 0, (name, k[".vgpr_count"])
+
+
+@pytest.mark.parametrize("K", [2, 3, 4, 5])
+@pytest.mark.parametrize("slots,waves", [(16, 8), (32, 6), (64, 4)])
+def test_chain_gemm_fits_without_spills(kernels, K, slots, waves):
+    """The chain GEMM's loops are bound by issue: a register spilled is a scratch reload in every tile row."""
+    k = kernels["xg_gemm_kernel<%d, %d>" % (K, slots)]
+    assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0 and _waves(k) >= waves
