@@ -606,7 +606,10 @@ int gfl_register_layer(gfl_ctx* c, int li, int E, int H, int I, int k_gate, int 
     L.shared = 0;
     // the workspaces of calls of up to MAX_PICKS picks for this shape, reserved now so that no such call allocates
     if (const int r = reserve_ws(c, H, I)) return r;
-    return reserve_chains(c, L);
+    const int r = reserve_chains(c, L);
+    if (r != GFL_ENOMEM) return r;
+    g_err.clear();   // the layer is registered: without memory for the chains such calls keep the decode launches
+    return GFL_OK;
 }
 
 int gfl_register_shared(gfl_ctx* c, int li, int k_gate, int k_up, int k_down, const uint64_t* ptr_row)
@@ -639,6 +642,29 @@ int gfl_register_shared(gfl_ctx* c, int li, int k_gate, int k_up, int k_down, co
     return GFL_OK;
 }
 
+// Sizes of the prefill workspace for P picks of M tokens over E experts: the plan's ints, then the data of each path.
+struct GwsSizes
+{
+    size_t n_it, ints;              // GEMM items; bytes of the plan
+    size_t g_xt, g_ygu, g_xd, g_yr; // MFMA grouped path
+    size_t c_xt, c_ygu, c_xd, c_yr; // EXACT chains
+    size_t total() const { return ints + std::max(g_xt + g_ygu + g_xd + g_yr, c_xt + c_ygu + c_xd + c_yr); }
+};
+
+static GwsSizes gws_sizes(int P, int M, int E, int H, int I)
+{
+    GwsSizes z;
+    const size_t nch = (P + gfl::GP_PLAN_CHUNK - 1) / gfl::GP_PLAN_CHUNK;
+    z.n_it = (size_t)gfl::gemm_items(P, E, gfl::GP_MIN_MT);
+    z.ints = align256(sizeof(int) * (4 + 4 * z.n_it + 2 * (size_t)P + (size_t)E + (E + 1) + 8 * (size_t)P + (size_t)M +
+                                     nch * (E + 1)));
+    z.g_xt = align256(2 * 2 * (size_t)P * H); z.g_ygu = align256(2 * 2 * (size_t)P * I);
+    z.g_xd = align256(2 * (size_t)P * I); z.g_yr = align256(2 * (size_t)P * H);
+    z.c_xt = align256(4 * 2 * (size_t)P * H); z.c_ygu = align256(2 * 2 * (size_t)P * I);
+    z.c_xd = align256(4 * (size_t)P * I); z.c_yr = align256(2 * (size_t)P * H);
+    return z;
+}
+
 static int run_chains(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64_t* sel, const void* w, int w_is_half,
                       int M, int topk, float* out, float act_limit, hipStream_t st);
 
@@ -654,21 +680,23 @@ static int run_chains(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64
 //     M = 27 181 -> 177
 //   E = 72: M = 9 [1] 259 -> 240, M = 64 [7.1] 1250 -> 526
 // The chains' combine writes 16 bytes at a time, and the forced launch shapes (GFL_SLOTS_PER_PASS, GFL_RELAY) name the
-// decode launches, so an unaligned out and a context with either keep those.
-static bool takes_chains(const gfl_ctx* c, const Layer& L, int P, int mode, const float* out)
+// decode launches, so an unaligned out and a context with either keep those; so does one whose registration found no memory
+// for the chains' workspace.
+static bool takes_chains(const gfl_ctx* c, const Layer& L, int M, int topk, int mode, const float* out)
 {
+    const int P = M * topk;
     if (mode == GFL_MODE_MFMA) return false;
     if (P > gfl::MAX_PICKS) return true;
     const bool enough = L.K[0] == L.K[1] ? 2 * P >= L.E : 4 * P >= 3 * L.E;
     return P > 64 && enough && !(reinterpret_cast<uintptr_t>(out) & 15) && c->ns_override == 0 &&
-           c->rw_override[0] < 0;
+           c->rw_override[0] < 0 && gws_sizes(P, M, L.E, L.H, L.I).total() <= c->gws_bytes;
 }
 
 // A call of picks on the launches that suit it (caller holds c->mu, device set; arguments checked).
 static int forward_picks(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64_t* sel, const void* w, int w_is_half,
                          int M, int topk, float* out, int mode, float act_limit, hipStream_t st, const char* who)
 {
-    if (takes_chains(c, L, M * topk, mode, out))
+    if (takes_chains(c, L, M, topk, mode, out))
         return run_chains(c, L, x, sel, w, w_is_half, M, topk, out, act_limit, st);
     if (!c->ws || L.H > c->ws_H || L.I > c->ws_I) return fail(GFL_ERUNTIME, std::string(who) + ": workspace not reserved");
     Workspace ws;
@@ -767,7 +795,11 @@ static int grow(gfl_ctx* c, hipStream_t st, void** buf, size_t* have, size_t nee
                                                   "(gfl_grouped_reserve, or one call of this shape first)");
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, need);
-    if (e != hipSuccess) return fail(GFL_ENOMEM, std::string(who) + ": workspace hipMalloc: " + hipGetErrorString(e));
+    if (e != hipSuccess)
+    {
+        (void)hipGetLastError();   // reported here, not by the next launch's check
+        return fail(GFL_ENOMEM, std::string(who) + ": workspace hipMalloc: " + hipGetErrorString(e));
+    }
     if (zero && (e = hipMemset(p, 0, need)) != hipSuccess)
     {
         hipFree(p);
@@ -782,23 +814,15 @@ static int grow(gfl_ctx* c, hipStream_t st, void** buf, size_t* have, size_t nee
 
 static int grouped_workspace(gfl_ctx* c, hipStream_t st, int P, int M, int E, int H, int I, const char* who, Gws& w)
 {
-    const size_t nch = (P + gfl::GP_PLAN_CHUNK - 1) / gfl::GP_PLAN_CHUNK;
-    const size_t n_it = (size_t)gfl::gemm_items(P, E, gfl::GP_MIN_MT);
-    const size_t n_int = 4 + 4 * n_it + 2 * (size_t)P + (size_t)E + (E + 1) + 8 * (size_t)P + (size_t)M + nch * (E + 1);
-    const size_t b_int = align256(sizeof(int) * n_int);
-    const size_t g_xt = align256(2 * 2 * (size_t)P * H), g_ygu = align256(2 * 2 * (size_t)P * I);
-    const size_t g_xd = align256(2 * (size_t)P * I), g_yr = align256(2 * (size_t)P * H);
-    const size_t c_xt = align256(4 * 2 * (size_t)P * H), c_ygu = align256(2 * 2 * (size_t)P * I);
-    const size_t c_xd = align256(4 * (size_t)P * I), c_yr = align256(2 * (size_t)P * H);
-    const size_t data = std::max(g_xt + g_ygu + g_xd + g_yr, c_xt + c_ygu + c_xd + c_yr);
-    if (const int r = grow(c, st, &c->gws, &c->gws_bytes, b_int + data, false, who)) return r;
+    const GwsSizes z = gws_sizes(P, M, E, H, I);
+    if (const int r = grow(c, st, &c->gws, &c->gws_bytes, z.total(), false, who)) return r;
     char* b = static_cast<char*>(c->gws);
     int* ip = reinterpret_cast<int*>(b);
     gfl::GPlan& gp = w.gp;
     gp.hdr = ip;
     gp.item = reinterpret_cast<int4*>(gp.hdr + 4);
-    gp.tok_svh = reinterpret_cast<uint64_t*>(gp.item + n_it);
-    gp.cnt = gp.hdr + 4 + 4 * n_it + 2 * (size_t)P;
+    gp.tok_svh = reinterpret_cast<uint64_t*>(gp.item + z.n_it);
+    gp.cnt = gp.hdr + 4 + 4 * z.n_it + 2 * (size_t)P;
     gp.off = gp.cnt + E;
     gp.slot_pick = gp.off + E + 1;
     gp.slot_e = gp.slot_pick + P;
@@ -809,15 +833,15 @@ static int grouped_workspace(gfl_ctx* c, hipStream_t st, int P, int M, int E, in
     gp.tok_w = reinterpret_cast<float*>(gp.tok_slot + P);
     gp.tok_npk = reinterpret_cast<int*>(gp.tok_w + P);
     gp.ccnt = gp.tok_npk + M;
-    char* d = b + b_int;
+    char* d = b + z.ints;
     w.xt = reinterpret_cast<uint16_t*>(d);
-    w.ygu16 = reinterpret_cast<uint16_t*>(d + g_xt);
-    w.xd = reinterpret_cast<uint16_t*>(d + g_xt + g_ygu);
-    w.yraw = reinterpret_cast<uint16_t*>(d + g_xt + g_ygu + g_xd);
+    w.ygu16 = reinterpret_cast<uint16_t*>(d + z.g_xt);
+    w.xd = reinterpret_cast<uint16_t*>(d + z.g_xt + z.g_ygu);
+    w.yraw = reinterpret_cast<uint16_t*>(d + z.g_xt + z.g_ygu + z.g_xd);
     w.xte = reinterpret_cast<float*>(d);
-    w.ygue = reinterpret_cast<uint16_t*>(d + c_xt);
-    w.xde = reinterpret_cast<float*>(d + c_xt + c_ygu);
-    w.yre = reinterpret_cast<uint16_t*>(d + c_xt + c_ygu + c_xd);
+    w.ygue = reinterpret_cast<uint16_t*>(d + z.c_xt);
+    w.xde = reinterpret_cast<float*>(d + z.c_xt + z.c_ygu);
+    w.yre = reinterpret_cast<uint16_t*>(d + z.c_xt + z.c_ygu + z.c_xd);
     return GFL_OK;
 }
 

@@ -96,7 +96,8 @@ int gfl_ctx_check(gfl_ctx* ctx);
 int gfl_register_layer(gfl_ctx* ctx, int li, int E, int H, int I, int k_gate, int k_up, int k_down,
                        const uint64_t* ptrs);
 /* (Registration also reserves the decode and prefill workspaces for 1024 picks at the largest registered sizes, so that
- * gfl_moe_forward never allocates up to 1024 picks.) */
+ * gfl_moe_forward never allocates up to 1024 picks. Where there is no memory for the prefill workspace, the layer is
+ * registered all the same, and gfl_moe_forward keeps its calls of up to 1024 picks on the decode launches.) */
 
 /* Shape of a registered layer: info[6] = {E, H, I, k_gate, k_up, k_down} (host array). The forward calls take no
  * shape arguments, so callers check their x / out widths against H with it (tier_forward checks x.size(1) == H,

@@ -1,0 +1,77 @@
+"""Which kernels a forward call launches, on the CPU: the built library runs against hip_recorder.c instead of the HIP
+runtime. All launch shapes are bit-identical by design, so no output tells which of them ran."""
+import json
+import os
+import re
+import subprocess
+import sys
+
+import pytest
+
+from conftest import PKG
+
+DRIVER = r"""
+import ctypes as C, json, sys
+rec = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+rec.hip_recorder_log.restype = C.c_char_p
+rec.hip_recorder_limit.argtypes = [C.c_size_t]
+import _native
+lib, job, h = _native.load(), json.load(sys.stdin), C.c_void_p()
+_native.check(lib.gfl_ctx_create(0, C.byref(h)))
+if job["limit"] is not None:
+    rec.hip_recorder_limit(job["limit"])
+E, H, I, Ks = job["layer"]
+rc = lib.gfl_register_layer(h, 0, E, H, I, *Ks, (C.c_uint64 * (9 * E))(*[1 << 20] * (9 * E)))
+out = [[rc, lib.gfl_last_error().decode(), ""]]
+rec.hip_recorder_limit(C.c_size_t(-1).value)
+for M, topk, mode, offset in job["calls"]:
+    rec.hip_recorder_clear()
+    if mode == "grouped":
+        rc = lib.gfl_grouped_forward(h, 0, 1 << 21, 1 << 22, 1 << 23, 1, M, topk, 1 << 24, 0.0, None)
+    elif mode == "reserve":
+        rc = lib.gfl_grouped_reserve(h, M * topk)
+    else:
+        rc = lib.gfl_moe_forward(h, 0, 1 << 21, 1 << 22, 1 << 23, 1, M, topk, (1 << 24) + offset, mode, 0.0, None)
+    out.append([rc, lib.gfl_last_error().decode(), rec.hip_recorder_log().decode()])
+print(json.dumps(out))
+"""
+
+
+@pytest.fixture(scope="module")
+def launches(tmp_path_factory):
+    """launches(layer, calls, limit, env): [(rc, error, [kernel names])] of the registration and of each call
+    (M, topk, mode, offset of out), on a context created with env and `limit` bytes of device memory left after that."""
+    import _native
+    if not os.path.exists(_native.LIB_PATH):
+        pytest.skip("library not built")
+    so = str(tmp_path_factory.mktemp("rec") / "hip_recorder.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-o", so,
+                    os.path.join(os.path.dirname(__file__), "hip_recorder.c")], check=True)
+
+    def run(layer, calls, limit=None, env=()):
+        r = subprocess.run([sys.executable, "-c", DRIVER, so], input=json.dumps(dict(layer=layer, calls=calls, limit=limit)),
+                           capture_output=True, text=True, env=dict(os.environ, PYTHONPATH=PKG, **dict(env)))
+        assert r.returncode == 0, r.stderr[-2000:]
+        got = json.loads(r.stdout.strip().split("\n")[-1])
+        names = subprocess.run(["c++filt"], input="\n".join(g[2].replace("\n", " ") for g in got), capture_output=True,
+                               text=True, check=True).stdout.split("\n")
+        return [(rc, err, re.findall(r"(?:gfl::)(\w+(?:<[^(]*>)?)\(", n)) for (rc, err, _), n in zip(got, names)]
+    return run
+
+
+EXACT, MFMA = 1, 3
+
+
+def test_registration_without_memory_for_the_chains(launches):
+    """Room for the decode workspace (28 MB at H = 4096, I = 256) but not for the chains' (44 MB): the layer is registered
+    and its calls run on the decode launches, none of them reporting the refused allocation; with memory they take the
+    chains."""
+    got = launches((8, 4096, 256, (3, 3, 3)), [(65, 1, EXACT, 0), (4, 4, EXACT, 0), (16, 16, "reserve", 0),
+                                              (65, 1, EXACT, 0), (256, 1, EXACT, 0), (512, 1, EXACT, 0)], limit=40 << 20)
+    assert [(rc, err) for rc, err, _ in got] == [(0, "")] * len(got)
+    assert got[1][2] == ["plan_kernel", "gu_kernel<3, 4, false>", "down_kernel<3, 4, false>"]
+    assert got[2][2] == ["gu_relay_kernel<3, 4>", "dn_relay_kernel<3, 1>"]
+    for k, slots in ((4, 32), (5, 64)):
+        assert got[k][2] == ["gp_plan_kernel", "gp_prep_kernel<true, false>", "xg_gemm_kernel<3, %d>" % slots,
+                             "gp_act_kernel<true, 1>", "xg_gemm_kernel<3, %d>" % slots, "gp_comb_kernel"]
+    assert got[6][2] == ["plan_kernel", "gu_kernel<3, 4, false>", "down_kernel<3, 4, false>"]   # beyond what was reserved
