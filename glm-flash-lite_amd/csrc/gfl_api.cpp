@@ -866,11 +866,12 @@ static int run_chains(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64
     Gws ws;
     if (const int rc = grouped_workspace(c, st, P, M, L.E, L.H, L.I, "gfl_moe_forward", ws)) return rc;
     auto gate_up = [&] {
-        return gfl::launch_chains_gate_up(L.dptrs, sel, w, w_is_half ? 1 : 0, P, topk, L.E, L.H, L.I, L.K[0], L.K[1], x,
-                                          ws.gp, P, ws.xte, ws.ygue, ws.xde, c->silu_tab, act_limit, st);
+        return gfl::launch_chains_gate_up(L.dptrs, sel, w, w_is_half ? 1 : 0, P, topk, L.E, L.H, L.I, L.K[0], L.K[1],
+                                          L.K[2], x, ws.gp, P, ws.xte, ws.ygue, ws.xde, c->silu_tab, act_limit, st);
     };
     auto down = [&] {
-        return gfl::launch_chains_down(L.dptrs, P, topk, L.E, L.H, L.I, L.K[2], ws.gp, P, ws.xde, ws.yre, out, st);
+        return gfl::launch_chains_down(L.dptrs, P, topk, L.E, L.H, L.I, L.K[0], L.K[1], L.K[2], ws.gp, P, ws.xde, ws.yre, out,
+                                       st);
     };
     // up to MAX_PICKS picks the stages are the decode launches' (1 gate|up, 3 down); above, the call is one stage
     int r;

@@ -141,10 +141,10 @@ size_t grouped_gemm_lds_bytes(int K);
 // order. xt [2][cap][H] fp32, ygu [2][cap][I] fp16, xd [cap][I] fp32, yraw [cap][H] fp16 workspace, cap >= P,
 // cap * max(H, I) * 4 < 2^31 (else -1, nothing launched).
 int launch_chains_gate_up(const uint64_t* ptrs, const int64_t* sel, const void* w, int w_half, int P, int topk, int E,
-                          int H, int I, int Kg, int Ku, const uint16_t* x, const GPlan& g, int cap, float* xt,
+                          int H, int I, int Kg, int Ku, int Kd, const uint16_t* x, const GPlan& g, int cap, float* xt,
                           uint16_t* ygu, float* xd, const float* silu_tab, float act_limit, hipStream_t st);
-int launch_chains_down(const uint64_t* ptrs, int P, int topk, int E, int H, int I, int Kd, const GPlan& g, int cap,
-                       const float* xd, uint16_t* yraw, float* out, hipStream_t st);
+int launch_chains_down(const uint64_t* ptrs, int P, int topk, int E, int H, int I, int Kg, int Ku, int Kd, const GPlan& g,
+                       int cap, const float* xd, uint16_t* yraw, float* out, hipStream_t st);
 // The grouped plan alone (first three launches of launch_grouped): slots, offsets, job order per token.
 // ptrs may be NULL (tok_svh is then 0).
 void launch_grouped_plan(const uint64_t* ptrs, const int64_t* sel, const void* w, int w_half, int P, int topk, int E,

@@ -1383,14 +1383,21 @@ static int xg_gemm_launch(const XgArgs& a, int nmat, hipStream_t st)
     return 0;
 }
 
-// Slots per pass of a call of P picks over E experts: the smallest pass that holds an expert's mean share, since a
-// smaller pass leaves more waves per SIMD and a larger one decodes an expert's weights less often. Measured at E = 288,
-// top-8 (ms per layer with 16 / 32 / 64; P / E in brackets): M = 64 [1.8] 1.05 / 1.07 / 1.27, M = 333 [9.3] 1.62 / 1.64 /
-// 1.80, M = 500 [14] 2.75 / 2.59 / 2.77, M = 700 [19] 3.71 / 3.12 / 3.35, M = 1024 [28] 5.05 / 4.21 / 4.22, M = 2048 [57]
-// 9.39 / 7.84 / 7.07.
-static int xg_slots(int P, int E)
+// Slots per pass of a call of P picks over E experts: 16 below 8 picks per expert, 32 below 28, else 64. A smaller pass leaves
+// more waves per SIMD, a larger one decodes an expert's weights less often. Measured at E = 288, top-8, 3 bits (ms per layer
+// with 16 / 32 / 64; P / E in brackets): M = 64 [1.8] 1.05 / 1.07 / 1.27, M = 333 [9.3] 1.62 / 1.64 / 1.80, M = 500 [14] 2.75 /
+// 2.59 / 2.77, M = 700 [19] 3.71 / 3.12 / 3.35, M = 1024 [28] 5.05 / 4.21 / 4.22, M = 2048 [57] 9.39 / 7.84 / 7.07.
+// With 5 bits a 64-slot pass takes 84 KB of LDS, one workgroup per CU (2 waves per SIMD): where all three matrices have 5, 32
+// slots from 28 picks on too, and where two have, below 48 picks (64 -> 32 slots, ms; bits gate/up/down): 5/5/5 M = 1024 5.55
+// -> 4.56, M = 1500 6.83 -> 6.54, M = 2048 8.68 -> 8.34, M = 4096 16.7 -> 15.6, E = 72 M = 300 [33] 1.63 -> 1.41, M = 1200 [133]
+// 5.07 -> 4.62, H = 4096 I = 2048 M = 2048 9.26 -> 8.78; 5/5/3 M = 1024 5.14 -> 4.40, M = 1500 [42] 6.45 -> 6.40, M = 2048 8.13
+// -> 8.13 and 8.13 -> 8.22, M = 4096 [114] 15.8 -> 15.5; 5/2/5 M = 1024 5.26 -> 4.41, M = 1500 6.56 -> 6.43, M = 2048 8.24 ->
+// 8.17 and 8.21 -> 8.21. With one matrix of 5 bits 64 stays: 3/3/5 M = 1500 5.99 -> 6.33, M = 2048 7.72 -> 8.08, M = 4096 15.1
+// -> 15.4 (but M = 1024 4.72 -> 4.37); 3/5/4 M = 2048 7.74 -> 8.13.
+static int xg_slots(int P, int E, int Kg, int Ku, int Kd)
 {
-    return P < 8 * E ? 16 : P < 28 * E ? 32 : XG_MS;
+    const int five = (Kg == 5) + (Ku == 5) + (Kd == 5);
+    return P < 8 * E ? 16 : P < 28 * E || five == 3 || (five == 2 && P < 48 * E) ? 32 : XG_MS;
 }
 
 template <int K>
@@ -1507,12 +1514,12 @@ int launch_grouped(const uint64_t* ptrs, const int64_t* sel, const void* w, int 
 }
 
 int launch_chains_gate_up(const uint64_t* ptrs, const int64_t* sel, const void* w, int w_half, int P, int topk, int E,
-                          int H, int I, int Kg, int Ku, const uint16_t* x, const GPlan& g, int cap, float* xt,
-                          uint16_t* ygu, float* xd, const float* silu_tab, float act_limit, hipStream_t st)
+                          int H, int I, int Kg, int Ku, int Kd, const uint16_t* x, const GPlan& g, int cap,
+                          float* xt, uint16_t* ygu, float* xd, const float* silu_tab, float act_limit, hipStream_t st)
 {
     // the chain GEMM addresses its fp32 inputs with 32-bit byte offsets
     if ((size_t)cap * (size_t)(H > I ? H : I) * 4 > (size_t)0x7fffffff) return -1;
-    const int ms = xg_slots(P, E);
+    const int ms = xg_slots(P, E, Kg, Ku, Kd);
     launch_grouped_plan(ptrs, sel, w, w_half, P, topk, E, ms, g, st);
     const int parts = prep_parts(P, H);
     hipLaunchKernelGGL((gp_prep_kernel<true, false>), dim3((unsigned)(((long)P * parts + GP_TW - 1) / GP_TW)), dim3(GP_TW * 64), 0, st,
@@ -1536,10 +1543,10 @@ int launch_chains_gate_up(const uint64_t* ptrs, const int64_t* sel, const void* 
     return 0;
 }
 
-int launch_chains_down(const uint64_t* ptrs, int P, int topk, int E, int H, int I, int Kd, const GPlan& g, int cap,
-                       const float* xd, uint16_t* yraw, float* out, hipStream_t st)
+int launch_chains_down(const uint64_t* ptrs, int P, int topk, int E, int H, int I, int Kg, int Ku, int Kd, const GPlan& g,
+                       int cap, const float* xd, uint16_t* yraw, float* out, hipStream_t st)
 {
-    const int ms = xg_slots(P, E);
+    const int ms = xg_slots(P, E, Kg, Ku, Kd);
     XgArgs a;
     a.ptrs = ptrs; a.mat_base = 2; a.kdim = I; a.ndim = H; a.cap = cap; a.nit = gemm_items(P, E, ms); a.g = g;
     a.xin = xd; a.yout = yraw;

@@ -60,6 +60,33 @@ def launches(tmp_path_factory):
 
 
 EXACT, MFMA = 1, 3
+B, S = (5120, 1536, (3, 3, 3)), (512, 256, (3, 3, 3))   # the benchmark's layer, the GPU tests' small one
+
+
+@pytest.mark.parametrize("layer,call,env,first", [
+    # the calls of tests/test_gpu_parity.py that name their launches
+    ((108, *B), (16, 8, EXACT, 0), {}, "gp_plan"), ((169, *B), (32, 8, EXACT, 0), {}, "gp_plan"),
+    ((249, *B), (64, 8, EXACT, 0), {}, "gp_plan"),
+    ((288, *B), (16, 8, EXACT, 0), {}, "plan"), ((249, *B), (64, 8, EXACT, 4), {}, "plan"),
+    ((32, *S), (128, 8, EXACT, 0), {}, "gp_plan"), ((32, *S), (128, 8, EXACT, 4), {}, "plan"),
+    ((8, *S), (16, 8, EXACT, 0), {}, "gp_plan"), ((8, *S), (16, 8, EXACT, 4), {}, "plan"),
+    ((20, 512, 256, (3, 4, 3)), (8, 16, EXACT, 0), {}, "gp_plan"),
+    ((288, 512, 256, (3, 4, 3)), (8, 16, EXACT, 0), {}, "plan"),
+    ((20, 512, 256, (3, 4, 3)), (8, 16, EXACT, 0), {"GFL_RELAY": "1,1"}, "plan"),
+    ((6, *S), (12, 8, EXACT, 0), {"GFL_SLOTS_PER_PASS": "2"}, "plan"),
+    # either side of each line: 64 picks; half a pick per expert, three quarters where gate and up differ; mode; 1,024 picks
+    ((16, *S), (64, 1, EXACT, 0), {}, "gu"), ((16, *S), (8, 8, EXACT, 0), {}, "gu_relay"),
+    ((16, *S), (65, 1, EXACT, 0), {}, "gp_plan"),
+    ((130, *S), (65, 1, EXACT, 0), {}, "gp_plan"), ((131, *S), (65, 1, EXACT, 0), {}, "plan"),
+    ((88, 512, 256, (3, 4, 3)), (66, 1, EXACT, 0), {}, "gp_plan"), ((89, 512, 256, (3, 4, 3)), (66, 1, EXACT, 0), {}, "plan"),
+    ((16, *S), (65, 1, MFMA, 0), {}, "plan"),
+    ((1024, *S), (1025, 1, EXACT, 0), {}, "gp_rank"), ((16, *S), (4, 16, "grouped", 0), {}, "gp_plan"),
+])
+def test_launch_choice(launches, layer, call, env, first):
+    """The first kernel of a call: relay or per-slot / per-entry decode launches (plan_kernel above 64 picks), or the grouped
+    plan of the chains and the grouped path."""
+    (rc, err, _), (crc, cerr, names) = launches(layer, [call], env=env)
+    assert (rc, err, crc, cerr) == (0, "", 0, "") and names[0].split("<")[0] == first + "_kernel", names
 
 
 def test_registration_without_memory_for_the_chains(launches):
@@ -75,3 +102,19 @@ def test_registration_without_memory_for_the_chains(launches):
         assert got[k][2] == ["gp_plan_kernel", "gp_prep_kernel<true, false>", "xg_gemm_kernel<3, %d>" % slots,
                              "gp_act_kernel<true, 1>", "xg_gemm_kernel<3, %d>" % slots, "gp_comb_kernel"]
     assert got[6][2] == ["plan_kernel", "gu_kernel<3, 4, false>", "down_kernel<3, 4, false>"]   # beyond what was reserved
+
+
+@pytest.mark.parametrize("Ks,M,slots", [
+    ((3, 3, 3), 7, 16), ((3, 3, 3), 8, 32), ((3, 3, 3), 27, 32), ((3, 3, 3), 28, 64), ((5, 3, 4), 28, 64),
+    ((3, 3, 5), 200, 64), ((5, 5, 5), 7, 16), ((5, 5, 2), 27, 32), ((5, 5, 2), 28, 32), ((5, 2, 5), 47, 32),
+    ((4, 5, 5), 48, 64), ((5, 5, 5), 60, 32), ((5, 5, 5), 200, 32),
+])
+def test_chain_pass_sizes(launches, Ks, M, slots):
+    """16, 32 and 64 slots per pass by picks per expert; with matrices of 5 bits, whose 64-slot pass leaves a CU one
+    workgroup, 32 for longer. Calls within 1,024 picks and above take the same sizes."""
+    for E in (16, 288):
+        (rc, err, _), call = launches((E, 512, 256, Ks), [(M * E // 16, 16, EXACT, 0)])
+        assert (rc, err, call[0], call[1]) == (0, "", 0, "")
+        gemms = [n for n in call[2] if n.startswith("xg_gemm_kernel")]
+        want = ["xg_gemm_kernel<%d, %d>" % (k, slots) for k in (Ks if Ks[0] != Ks[1] else Ks[1:])]
+        assert gemms == want, call[2]
