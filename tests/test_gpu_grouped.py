@@ -114,7 +114,7 @@ def test_grouped_mixed_k(gpu, oracle, Ks):
 
 @pytest.mark.gpu
 def test_grouped_config_shape_vs_decode_path(gpu):
-    """Config-1 shape (H=5120, I=1536, K=3, top-8 of 288), M=128: against the bit-exact decode path on the GPU."""
+    """Config-1 shape (H=5120, I=1536, K=3, top-8 of 288), M=128: against the bit-exact path on the GPU."""
     import synth
     H, I, E = 5120, 1536, 288
     _layer(gpu, 24, E, H, I)

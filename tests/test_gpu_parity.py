@@ -30,12 +30,20 @@ def _host_experts(oracle, L):
     return ex
 
 
-def _forward(gpu, li, x16, sel, w, w_half=False):
+def _register_repeated(gpu, li, L, E):
+    """Register li as E experts, those of L repeated: more experts than a call's picks reach keep calls of 65..1,024 picks
+    on the decode launches (tests/test_launches.py)."""
+    gpu.register_layer(li, E, L.H, L.I, L.Ks, (L.ptr_table * (E // L.E + 1))[:9 * E], keep=L)
+
+
+def _forward(gpu, li, x16, sel, w, w_half=False, offset=0):
+    """offset: bytes by which out lies off 16-byte alignment (4: calls of 65..1,024 picks keep the decode launches)."""
     import torch
     xd = torch.from_numpy(x16.view(np.int16)).view(torch.float16).cuda()
     seld = torch.from_numpy(np.ascontiguousarray(sel, dtype=np.int64)).cuda()
     wd = torch.from_numpy(np.ascontiguousarray(w)).cuda()
-    out = torch.empty(x16.shape, dtype=torch.float32, device="cuda")
+    buf = torch.empty(x16.size + 4, dtype=torch.float32, device="cuda")
+    out = buf[offset // 4:offset // 4 + x16.size].view(x16.shape)
     gpu.moe_forward(li, xd.contiguous(), seld, wd, out)
     torch.cuda.synchronize()
     return out.cpu().numpy()
@@ -116,10 +124,12 @@ def test_forward_equals_reference_engine_golden(gpu, nt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("offset", [0, 4])
 @pytest.mark.parametrize("scale", [0.35, 0.05, 1.0])
-def test_forward_sweep_bitexact(gpu, oracle, scale):
+def test_forward_sweep_bitexact(gpu, oracle, scale, offset):
     """16 tokens x every expert of an 8-expert layer (128 picks, 16 slots per expert): exercises many rounding ties,
-    small activations (fp16 subnormal range after the input Hadamard) and multi-pass slot chunks."""
+    small activations (fp16 subnormal range after the input Hadamard) and, with an out that is not 16-byte aligned, the
+    decode launches' multi-pass slot chunks (else the chain GEMMs)."""
     H, I, E = 512, 256, 8
     L = _layer(gpu, 5, E, H, I)
     ex = _host_experts(oracle, L)
@@ -127,9 +137,9 @@ def test_forward_sweep_bitexact(gpu, oracle, scale):
     x16 = (rng.standard_normal((16, H)) * scale).astype(np.float16)
     sel = np.tile(np.arange(E, dtype=np.int64), (16, 1))
     w = rng.random(sel.shape).astype(np.float32)
-    got = _forward(gpu, 5, x16, sel, w)
+    got = _forward(gpu, 5, x16, sel, w, offset=offset)
     want = oracle.moe_forward(ex, x16.astype(np.float32), sel, w, mode=1)
-    mx, rms, nbad = _report(f"sweep scale={scale}", got, want)
+    mx, rms, nbad = _report(f"sweep scale={scale} offset={offset}", got, want)
     assert nbad == 0
 
 
@@ -271,8 +281,10 @@ def test_forward_slots_per_pass_bitexact(gpu, oracle, ns):
 
 
 @pytest.mark.gpu
-def test_forward_max_picks_bitexact(gpu, oracle):
-    """The largest decode call: 128 tokens x top-8 = 1024 picks over 32 experts (every expert in several jobs)."""
+@pytest.mark.parametrize("offset", [0, 4])
+def test_forward_max_picks_bitexact(gpu, oracle, offset):
+    """128 tokens x top-8 = 1024 picks over 32 experts (every expert in several jobs): the largest call of the one-launch
+    plan on the chain GEMMs and, with an out that is not 16-byte aligned, of the decode launches."""
     H, I, E = 512, 256, 32
     L = _layer(gpu, 9, E, H, I)
     ex = _host_experts(oracle, L)
@@ -281,9 +293,9 @@ def test_forward_max_picks_bitexact(gpu, oracle):
     x16 = (rng.standard_normal((M, H)) * 0.5).astype(np.float16)
     sel = np.stack([rng.permutation(E)[:8] for _ in range(M)]).astype(np.int64)
     w = rng.random(sel.shape).astype(np.float32)
-    got = _forward(gpu, 9, x16, sel, w)
+    got = _forward(gpu, 9, x16, sel, w, offset=offset)
     want = oracle.moe_forward(ex, x16.astype(np.float32), sel, w, mode=1)
-    mx, rms, nbad = _report("max picks", got, want)
+    mx, rms, nbad = _report(f"max picks offset={offset}", got, want)
     assert nbad == 0
 
 
@@ -336,21 +348,25 @@ def test_config2_full_shape_bitexact(gpu, oracle, layer_kind, M):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M", [16, 32, 64])
-def test_config3_full_shape_bitexact(gpu, oracle, M):
+@pytest.mark.parametrize("M,table,offset", [(16, 0, 0), (32, 0, 0), (64, 0, 0), (16, 288, 0), (64, 0, 4)],
+                         ids=["16", "32", "64", "16-decode-launches", "64-decode-launches"])
+def test_config3_full_shape_bitexact(gpu, oracle, M, table, offset):
     """Config 3 at its shape: M = 16, 32 and 64 tokens, each routed top-8 over 288 experts with uniform N(0,1) logits,
-    H=5120, I=1536, 3 bpw, through the default launch choice (above 8 tokens: a workgroup per routed expert taking
-    its slots two per pass, gu_kernel / down_kernel with NS = 2). The layer holds the routed union (up to 240
-    experts, 2.1 GB); the oracle evaluates rows 0, M/2 and M-1 with the whole call's jobs (moe_forward_rows), so each
-    checked row's combine order is the full batch's."""
+    H=5120, I=1536, 3 bpw. The layer holds the routed union (up to 240 experts, 2.1 GB), so that by their picks per
+    registered expert these calls take the chain GEMMs. Registered as 288 experts (M = 16), or with an out that is not
+    16-byte aligned (M = 64), they take the decode launches: a workgroup per routed expert taking its slots two per pass
+    (plan_kernel, gu_kernel / down_kernel with NS = 2). The oracle evaluates rows 0, M/2 and M-1 with the whole call's jobs
+    (moe_forward_rows), so each checked row's combine order is the full batch's."""
     import synth
     from oracle import Mat
     H, I, E = 5120, 1536, 288
     rng = np.random.default_rng(3000 + M)
     (sel, w16), _ = synth.route_uniform(M, E, 8, rng)
     L, sel2 = _union_layer(gpu, 40 + M, sel, H, I, (3, 3, 3))
+    if table:
+        _register_repeated(gpu, 40 + M, L, table)
     x16 = rng.standard_normal((M, H)).astype(np.float16)
-    got = _forward(gpu, 40 + M, x16, sel2, w16)
+    got = _forward(gpu, 40 + M, x16, sel2, w16, offset=offset)
     rows = [0, M // 2, M - 1]
     need = {int(e) for r in rows for e in sel2[r] if e >= 0}
     dummy = None
@@ -556,15 +572,18 @@ def test_relay_launches_full_shape_bitexact(gpu, oracle, relay, prio):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("relay", [None, "1,1"])
-def test_one_slot_per_pass_above_64_picks_bitexact(gpu, oracle, relay):
+@pytest.mark.parametrize("relay,table", [(None, 0), ("1,1", 0), (None, 288)])
+def test_one_slot_per_pass_above_64_picks_bitexact(gpu, oracle, relay, table):
     """Top-16 at M = 5 and 8 (80 and 128 picks, one slot per pass): more picks than the relay down launch's combine
-    list holds (one per lane of a wave), so these calls keep the per-slot launches, under the default launch choice
-    and with the relay forced (GFL_RELAY applies up to 64 picks); every token's row bit-exact, including tokens past
-    the first 64 picks. At 64 picks (M = 4) the relay launches run."""
+    list holds (one per lane of a wave), so with few picks per registered expert (table) these calls keep the per-slot
+    launches, and with the relay forced as well (GFL_RELAY applies up to 64 picks); under the default launch choice on 20
+    experts they take the chain GEMMs. Every token's row bit-exact, including tokens past the first 64 picks. At 64 picks
+    (M = 4) the relay launches run."""
     ctx = gpu if relay is None else _ctx_with_env(GFL_RELAY=relay)
     H, I, E, li = 512, 256, 20, 54 if relay is None else 55
     L = _layer(ctx, li, E, H, I, (3, 4, 3))
+    if table:
+        _register_repeated(ctx, li, L, table)
     ex = _host_experts(oracle, L)
     for M in (4, 5, 8):
         rng = np.random.default_rng(5400 + M)
