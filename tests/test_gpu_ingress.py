@@ -199,6 +199,38 @@ def test_device_worker_refuses_and_answers(gpu, oracle, layer):
     assert int(ctrl[1].item()) == 7 and not torch.any(hout)
 
 
+@pytest.mark.parametrize("offset", [0, 4])
+def test_device_worker_batched_jobs_bitexact(gpu, oracle, layer, offset):
+    """Jobs of up to 16 x 8 picks, which the worker computes on the chain GEMMs (with an hout that is not 16-byte aligned,
+    on the decode launches): full, with few picks, with none, from fewer tokens; then nothing pending."""
+    import torch
+    bsz = 16
+    rng = np.random.default_rng(91 + offset)
+    x = rng.standard_normal((bsz, H)).astype(np.float16)
+    hx = torch.from_numpy(x).cuda()
+    buf = torch.empty(bsz * H + 4, dtype=torch.float32, device="cuda")
+    hout = buf[offset // 4:offset // 4 + bsz * H]
+    ctrl = torch.zeros(16, dtype=torch.int64, device="cuda")
+    hp = torch.zeros(bsz * 8 * 3, dtype=torch.int32, device="cuda")
+    full = [(t, int(e), float(rng.random())) for t in range(bsz) for e in rng.permutation(E)[:8]]
+    for seq, (picks, ntok) in enumerate([(full, bsz), (full[3::17], bsz), ([], bsz), (full[:40], 5)], start=1):
+        bits = [(t, e, int(np.array([wv], np.float32).view(np.int32)[0])) for t, e, wv in picks]
+        hp[:3 * len(bits)] = torch.tensor(bits, dtype=torch.int32).reshape(-1).cuda()
+        ctrl.copy_(torch.tensor([seq, seq - 1, 71, ntok, len(bits)] + [0] * 11, dtype=torch.int64))
+        hout.fill_(float("nan"))
+        print(f"device worker: job {seq}, {len(bits)} picks of {ntok} tokens, offset {offset}", flush=True)
+        gpu.ingress_serve(71, bsz, 8, ctrl.data_ptr(), hx.data_ptr(), hp.data_ptr(), hout.data_ptr())
+        torch.cuda.synchronize()
+        gpu.check()
+        assert int(ctrl[1].item()) == seq
+        hs, hw = _host_selection(bits, len(bits), bsz)
+        want = oracle.moe_forward(_experts(layer), x.astype(np.float32), hs, hw, mode=1)
+        assert np.array_equal(hout.cpu().numpy().reshape(bsz, H), want)
+    gpu.ingress_serve(71, bsz, 8, ctrl.data_ptr(), hx.data_ptr(), hp.data_ptr(), hout.data_ptr())
+    torch.cuda.synchronize()
+    assert not torch.any(hout)
+
+
 def test_ctx_check_reports_expired_relay_waits(gpu, layer, monkeypatch):
     """A zero bound on the relay hand-off wait (GFL_RELAY_SPIN_LIMIT=0, set before the context is made) makes every
     wait expire at once; the kernels finish normally and gfl_ctx_check reports the expiries, then clears them. The
