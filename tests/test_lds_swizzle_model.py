@@ -1,7 +1,8 @@
 """Host model of the swizzled input rings of the chain GEMM (xg_gemm_kernel) and the wide grouped GEMM (gw_gemm_kernel),
-k_prefill.hip: every lane's source address and LDS destination as the kernels form them, checked so that each fragment
-read finds the 16 bytes meant for it, every read and write stays in its row, array and ring, and the reads of 8
-consecutive lanes lie in different banks. The constants are read from the source."""
+k_prefill.hip: a copy by hand of the formulas for every lane's source address and LDS destination, checked so that each
+fragment read finds the 16 bytes meant for it, every read and write stays in its row, array and ring, and the reads of 8
+consecutive lanes lie in different banks. XG_NW, XG_MS, GP_NW, GW_MT and GW_GR are read from the source; the formulas are
+not, so a change of the kernels' addressing has to be made here too (the GPU tests hold the kernels themselves)."""
 import os
 import re
 
