@@ -1793,16 +1793,6 @@ static int device_cus()
     return cus[dev];
 }
 
-// LDS to request for a launch of nwg equal workgroups that each need `need` bytes: at least enough that a CU holds
-// no more than ceil(nwg / CUs) of them. The relay kernels use few registers, so the dispatcher could otherwise put one
-// workgroup more on some CUs than on the rest, and those CUs set the launch's time.
-static size_t balanced_lds(size_t need, long nwg)
-{
-    const long cus = device_cus(), per_cu = (nwg + cus - 1) / cus;
-    const size_t cap = (size_t)LDS_LIMIT / (size_t)(per_cu + 1) + 16;
-    return cap > need && cap <= (size_t)LDS_LIMIT ? cap : need;
-}
-
 // Waves of a kernel that one SIMD holds at once, from its register count (512 VGPRs per lane, allocated in blocks of
 // 8; at most 8 waves).
 static int resident_waves(const void* kern)
@@ -1811,6 +1801,21 @@ static int resident_waves(const void* kern)
     if (hipFuncGetAttributes(&at, kern) != hipSuccess || at.numRegs <= 0) return 3;
     const int regs = (at.numRegs + 7) / 8 * 8;
     return std::min(8, 512 / regs);
+}
+
+// LDS to request for a relay launch of nwg equal workgroups of 4 waves that each need `need` bytes, of which a CU's registers
+// hold cap: at least enough that a CU holds no more than ceil(nwg / CUs) of them (the dispatcher could otherwise put one
+// workgroup more on some CUs than on the rest, and those CUs set the launch's time) and, where they do not all fit at once,
+// no more than 4: with more, a short last round runs almost alone, which shows on a card under sustained load, where the
+// clock falls with the issue rate. us per 4 layers, 6 resident -> 4: M = 3 with the shared expert at H = 4096 I = 2048 (27
+// workgroups for every 4 CUs) 492 -> 467, M = 4 558 -> 535, M = 5 677 -> 658 on a card that had throttled (with 5 resident
+// 479, 545, 659), 454 -> 455, 518 -> 521 and 635 -> 639 on a cool one. Rounds of equal size instead (10 workgroups as 5 + 5)
+// measured config 2's M = 4 523 against 508 throttled, and up to 1.5% faster at M = 5..8.
+static size_t balanced_lds(size_t need, long nwg, int cap)
+{
+    const long cus = device_cus(), per_cu = (nwg + cus - 1) / cus, held = per_cu > cap ? std::min(4, cap) : per_cu;
+    const size_t lds = (size_t)LDS_LIMIT / (size_t)(held + 1) + 16;
+    return lds > need && lds <= (size_t)LDS_LIMIT ? lds : need;
 }
 
 // Progress priority of a relay launch (chain_relay's prio): on when the launch puts more than one wave on a SIMD and
@@ -1834,10 +1839,10 @@ static void gu_relay_launch(const GuArgs& a, int nmat, hipStream_t st)
     static const bool opened = open_lds(kern);
     (void)opened;
     const long nwg = (long)(a.P + a.nsh) * (a.I / (16 * CW)) * nmat;   // GEMV workgroups (plus the publishing one)
-    const size_t lds = balanced_lds(gu_relay_lds<K>(a.H, a.P, a.E), nwg);
+    static const int cap = resident_waves(reinterpret_cast<const void*>(kern));
+    const size_t lds = balanced_lds(gu_relay_lds<K>(a.H, a.P, a.E), nwg, cap);
     GuArgs b = a;
     b.nmat_launch = nmat;
-    static const int cap = resident_waves(reinterpret_cast<const void*>(kern));
     b.prio = relay_prio(a.prio, nwg * GU_NW, cap);
     timed_launch(kern, dim3(8 + relay_blocks(nwg, RW)), dim3(GU_NW * 64), lds, st, b);
 }
@@ -1850,10 +1855,10 @@ static void dn_relay_launch(const DnArgs& a, int P, hipStream_t st)
     static const bool opened = open_lds(kern);
     (void)opened;
     const long nwg = (long)(P + a.nsh) * (a.H / (16 * CW));
-    const size_t lds = balanced_lds(dn_relay_lds<K>(a.I), nwg);
+    static const int cap = resident_waves(reinterpret_cast<const void*>(kern));
+    const size_t lds = balanced_lds(dn_relay_lds<K>(a.I), nwg, cap);
     DnArgs b = a;
     b.pv_picks = P;
-    static const int cap = resident_waves(reinterpret_cast<const void*>(kern));
     b.prio = relay_prio(a.prio, nwg * GU_NW, cap);
     timed_launch(kern, dim3(relay_blocks(nwg, RW)), dim3(GU_NW * 64), lds, st, b);
 }

@@ -1,5 +1,5 @@
 /* The HIP runtime functions libgfl_moe.so calls, as a recorder for the CPU: device memory is host memory that no kernel
- * touches (hip_recorder_limit bounds it), and each launch appends its kernel's name to a log. Loaded with RTLD_GLOBAL before
+ * touches (hip_recorder_limit bounds it), and each launch appends its kernel's name and dynamic LDS bytes to a log. Loaded with RTLD_GLOBAL before
  * the library, so that the library's own launch code runs against it. */
 #include <hip/hip_runtime_api.h>
 #include <stdio.h>
@@ -22,12 +22,13 @@ void hip_recorder_limit(size_t bytes) { left = bytes; }
 void hip_recorder_clear(void) { launches[log_len = 0] = 0; }
 const char* hip_recorder_log(void) { return launches; }
 
-static hipError_t launched(const void* fn)
+static hipError_t launched(const void* fn, size_t lds)
 {
     for (int i = 0; i < n_kernels; ++i)
         if (kernels[i].fn == fn)
         {
-            log_len += (size_t)snprintf(launches + log_len, sizeof launches - log_len, "%s\n", kernels[i].name);
+            log_len += (size_t)snprintf(launches + log_len, sizeof launches - log_len, "%s %zu\n", kernels[i].name,
+                                        lds);
             return done(log_len < sizeof launches ? hipSuccess : hipErrorOutOfMemory);
         }
     return done(hipErrorInvalidDeviceFunction);
@@ -66,7 +67,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, hipStream_t* s
 hipError_t hipLaunchKernel(const void* fn, dim3 g, dim3 b, void** args, size_t s, hipStream_t st)
 {
     (void)args; (void)st;
-    return g.x && g.y && g.z && b.x * b.y * b.z <= 1024 && s <= 163840 ? launched(fn) : done(hipErrorInvalidConfiguration);
+    return g.x && g.y && g.z && b.x * b.y * b.z <= 1024 && s <= 163840 ? launched(fn, s) : done(hipErrorInvalidConfiguration);
 }
 
 hipError_t hipMalloc(void** p, size_t n)

@@ -40,7 +40,8 @@ print(json.dumps(out))
 @pytest.fixture(scope="module")
 def launches(tmp_path_factory):
     """launches(layer, calls, limit, env): [(rc, error, [kernel names])] of the registration and of each call
-    (M, topk, mode, offset of out), on a context created with env and `limit` bytes of device memory left after that."""
+    (M, topk, mode, offset of out), on a context created with env and `limit` bytes of device memory left after that;
+    launches.lds has each launch's dynamic LDS bytes."""
     import _native
     if not os.path.exists(_native.LIB_PATH):
         pytest.skip("library not built")
@@ -55,6 +56,7 @@ def launches(tmp_path_factory):
         got = json.loads(r.stdout.strip().split("\n")[-1])
         names = subprocess.run(["c++filt"], input="\n".join(g[2].replace("\n", " ") for g in got), capture_output=True,
                                text=True, check=True).stdout.split("\n")
+        run.lds = [[int(v) for v in re.findall(r"\) (\d+)", n)] for n in names]
         return [(rc, err, re.findall(r"(?:gfl::)(\w+(?:<[^(]*>)?)\(", n)) for (rc, err, _), n in zip(got, names)]
     return run
 
@@ -118,3 +120,15 @@ def test_chain_pass_sizes(launches, Ks, M, slots):
         gemms = [n for n in call[2] if n.startswith("xg_gemm_kernel")]
         want = ["xg_gemm_kernel<%d, %d>" % (k, slots) for k in (Ks if Ks[0] != Ks[1] else Ks[1:])]
         assert gemms == want, call[2]
+
+
+@pytest.mark.parametrize("layer,M,per_cu", [
+    (B, 2, (3, 5)), (B, 3, (5, 4)), (B, 4, (6, 4)), (B, 8, (4, 4)),
+    ((4096, 2048, (3, 3, 3)), 3, (6, 6)), ((4096, 2048, (3, 3, 3)), 4, (4, 4)),
+])
+def test_relay_workgroups_per_cu(launches, layer, M, per_cu):
+    """The one-wave relay launches' LDS lets a CU (160 KB) hold the launch's share of workgroups where the registers take
+    that many (6), else 4."""
+    _, (rc, err, names) = launches((288, *layer), [(M, 8, EXACT, 0)])
+    assert (rc, err, names) == (0, "", ["gu_relay_kernel<3, 1>", "dn_relay_kernel<3, 1>"])
+    assert tuple(163840 // lds for lds in launches.lds[1]) == per_cu
