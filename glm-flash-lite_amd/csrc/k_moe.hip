@@ -1803,36 +1803,44 @@ static int resident_waves(const void* kern)
     return std::min(8, 512 / regs);
 }
 
-// LDS to request for a relay launch of nwg equal workgroups of 4 waves that each need `need` bytes, of which a CU's registers
-// hold cap: at least enough that a CU holds no more than ceil(nwg / CUs) of them (the dispatcher could otherwise put one
-// workgroup more on some CUs than on the rest, and those CUs set the launch's time) and, where they do not all fit at once,
-// no more than 4: with more, a short last round runs almost alone, which shows on a card under sustained load, where the
-// clock falls with the issue rate. us per 4 layers, 6 resident -> 4: M = 3 with the shared expert at H = 4096 I = 2048 (27
-// workgroups for every 4 CUs) 492 -> 467, M = 4 558 -> 535, M = 5 677 -> 658 on a card that had throttled (with 5 resident
-// 479, 545, 659), 454 -> 455, 518 -> 521 and 635 -> 639 on a cool one. Rounds of equal size instead (10 workgroups as 5 + 5)
-// measured config 2's M = 4 523 against 508 throttled, and up to 1.5% faster at M = 5..8.
-static size_t balanced_lds(size_t need, long nwg, int cap)
+// Workgroups (of 4 waves) that a CU is to hold of a relay launch of nwg equal ones, of which its registers take cap: its share,
+// and 4 where that is more than the registers take. With more than 4, a short last round runs almost alone, which shows on a
+// card under sustained load, where the clock falls with the issue rate. us per 4 layers, 6 held -> 4: M = 3 with the shared
+// expert at H = 4096 I = 2048 (27 workgroups for every 4 CUs) 492 -> 467, M = 4 558 -> 535, M = 5 677 -> 658 on a card that had
+// throttled (with 5 held 479, 545, 659), 454 -> 455, 518 -> 521 and 635 -> 639 on a cool one. Rounds of equal size instead (10
+// workgroups as 5 + 5) measured config 2's M = 4 523 against 508 throttled, and up to 1.5% faster at M = 5..8. beside (other GPU
+// work runs beside the call): 6 held would leave that work little room, so 4 from a share of 6 on (config 1 M = 4 with the
+// shared expert on a side stream, us per token: 40.7 -> 39.6).
+static int relay_held(long nwg, int cap, int beside)
 {
-    const long cus = device_cus(), per_cu = (nwg + cus - 1) / cus, held = per_cu > cap ? std::min(4, cap) : per_cu;
+    const long cus = device_cus(), share = (nwg + cus - 1) / cus;
+    return (int)(share > (beside ? std::min(5, cap) : cap) ? std::min(4, cap) : share);
+}
+
+// LDS to request so that a CU holds no more than `held` workgroups that each need `need` bytes: the relay kernels use few
+// registers, so the dispatcher could otherwise put one workgroup more on some CUs than on the rest, and those CUs set the
+// launch's time.
+static size_t balanced_lds(size_t need, int held)
+{
     const size_t lds = (size_t)LDS_LIMIT / (size_t)(held + 1) + 16;
     return lds > need && lds <= (size_t)LDS_LIMIT ? lds : need;
 }
 
 // Progress priority of a relay launch (chain_relay's prio): on when the launch puts more than one wave on a SIMD and
-// all of them fit at once (cap: resident_waves), so that a SIMD's last wave would otherwise run its last stretch
+// all of them run at once (held: relay_held), so that a SIMD's last wave would otherwise run its last stretch
 // alone. Measured on MI355X (config 1, us per token): M = 1 (gate|up 3 waves per SIMD of 3, down 2.5 of 4) 48.9 ->
 // 45.8; M = 2 with it on gate|up (3 of 4) 36.6 -> 34.9, while on a down launch of two rounds (5 waves per SIMD of 4) 0.4
 // slower; routed + shared expert in one call at M = 2 (gate|up 3.4 of 4) 42.4 -> 40.0. prio >= 0 (GFL_RELAY_PRIO)
 // forces it.
-static int relay_prio(int prio, long waves, int cap)
+static int relay_prio(int prio, long waves, int held)
 {
     if (prio >= 0) return prio;
     const long simds = 4L * device_cus();
-    return waves > simds && waves <= cap * simds ? 1 : 0;
+    return waves > simds && waves <= held * simds ? 1 : 0;
 }
 
 template <int K, int RW>
-static void gu_relay_launch(const GuArgs& a, int nmat, hipStream_t st)
+static void gu_relay_launch(const GuArgs& a, int nmat, int beside, hipStream_t st)
 {
     constexpr int CW = GU_NW / RW;
     auto kern = gu_relay_kernel<K, RW>;
@@ -1840,15 +1848,16 @@ static void gu_relay_launch(const GuArgs& a, int nmat, hipStream_t st)
     (void)opened;
     const long nwg = (long)(a.P + a.nsh) * (a.I / (16 * CW)) * nmat;   // GEMV workgroups (plus the publishing one)
     static const int cap = resident_waves(reinterpret_cast<const void*>(kern));
-    const size_t lds = balanced_lds(gu_relay_lds<K>(a.H, a.P, a.E), nwg, cap);
+    const int held = relay_held(nwg, cap, beside);
+    const size_t lds = balanced_lds(gu_relay_lds<K>(a.H, a.P, a.E), held);
     GuArgs b = a;
     b.nmat_launch = nmat;
-    b.prio = relay_prio(a.prio, nwg * GU_NW, cap);
+    b.prio = relay_prio(a.prio, nwg * GU_NW, held);
     timed_launch(kern, dim3(8 + relay_blocks(nwg, RW)), dim3(GU_NW * 64), lds, st, b);
 }
 
 template <int K, int RW>
-static void dn_relay_launch(const DnArgs& a, int P, hipStream_t st)
+static void dn_relay_launch(const DnArgs& a, int P, int beside, hipStream_t st)
 {
     constexpr int CW = GU_NW / RW;
     auto kern = dn_relay_kernel<K, RW>;
@@ -1856,10 +1865,11 @@ static void dn_relay_launch(const DnArgs& a, int P, hipStream_t st)
     (void)opened;
     const long nwg = (long)(P + a.nsh) * (a.H / (16 * CW));
     static const int cap = resident_waves(reinterpret_cast<const void*>(kern));
-    const size_t lds = balanced_lds(dn_relay_lds<K>(a.I), nwg, cap);
+    const int held = relay_held(nwg, cap, beside);
+    const size_t lds = balanced_lds(dn_relay_lds<K>(a.I), held);
     DnArgs b = a;
     b.pv_picks = P;
-    b.prio = relay_prio(a.prio, nwg * GU_NW, cap);
+    b.prio = relay_prio(a.prio, nwg * GU_NW, held);
     timed_launch(kern, dim3(relay_blocks(nwg, RW)), dim3(GU_NW * 64), lds, st, b);
 }
 
@@ -1911,7 +1921,7 @@ size_t down_lds_bytes(int K, int ns, int I, int P, int E, int mf, int rw)
 int launch_gate_up(int K, int ns, const uint64_t* ptrs, int mat_base, int nmat, const int64_t* sel, const void* w,
                    int w_half, int P, int topk, int E, int H, int I, int umax, const uint16_t* x, float* ygu,
                    uint16_t* xtd, int* act_cnt, const float* silu_tab, float act_limit, const PlanView& pv, float* out,
-                   int mf, int rw, int prio, int nsh, int gplan, int* status, int spin_max, hipStream_t st)
+                   int mf, int rw, int prio, int beside, int nsh, int gplan, int* status, int spin_max, hipStream_t st)
 {
     if (nsh && (!rw || mf)) return -1;   // shared-expert picks ride on the relay launches only
     GuArgs a;
@@ -1937,7 +1947,7 @@ int launch_gate_up(int K, int ns, const uint64_t* ptrs, int mat_base, int nmat, 
         // one slot per workgroup, slot = pick, rw waves per tile column
         a.nmat_total = 2 * (128 / (16 * (GU_NW / rw)));
         a.per_slot = 1;
-        GFL_K_SWITCH(K, GFL_RW_SWITCH(rw, (gu_relay_launch<K_, RW_>(a, nmat, st))))
+        GFL_K_SWITCH(K, GFL_RW_SWITCH(rw, (gu_relay_launch<K_, RW_>(a, nmat, beside, st))))
         return 0;
     }
     a.nmat_total = 2 * (128 / (16 * GU_NW));
@@ -1949,7 +1959,7 @@ int launch_gate_up(int K, int ns, const uint64_t* ptrs, int mat_base, int nmat, 
 
 int launch_down(int K, int ns, const uint64_t* ptrs, int topk, int H, int I, int umax, int P, int E, const int64_t* sel,
                 const void* w, int w_half, const PlanView& pv, const uint16_t* xtd, float* yd, int* out_cnt,
-                int* blk_cnt, float* out, int mf, int rw, int prio, int nsh, int* status, int spin_max,
+                int* blk_cnt, float* out, int mf, int rw, int prio, int beside, int nsh, int* status, int spin_max,
                 hipStream_t st)
 {
     if (nsh && (!rw || mf)) return -1;
@@ -1973,7 +1983,7 @@ int launch_down(int K, int ns, const uint64_t* ptrs, int topk, int H, int I, int
         // relay_combine_list holds the call's picks one per lane of a wave
         if (P > 64) return -1;
         a.per_slot = 1;
-        GFL_K_SWITCH(K, GFL_RW_SWITCH(rw, (dn_relay_launch<K_, RW_>(a, P, st))))
+        GFL_K_SWITCH(K, GFL_RW_SWITCH(rw, (dn_relay_launch<K_, RW_>(a, P, beside, st))))
         return 0;
     }
     a.per_slot = ns == 1;

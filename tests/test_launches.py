@@ -24,6 +24,7 @@ E, H, I, Ks = job["layer"]
 rc = lib.gfl_register_layer(h, 0, E, H, I, *Ks, (C.c_uint64 * (9 * E))(*[1 << 20] * (9 * E)))
 out = [[rc, lib.gfl_last_error().decode(), ""]]
 rec.hip_recorder_limit(C.c_size_t(-1).value)
+lib.gfl_ctx_set_shared(h, job["shared"])
 for M, topk, mode, offset in job["calls"]:
     rec.hip_recorder_clear()
     if mode == "grouped":
@@ -49,9 +50,9 @@ def launches(tmp_path_factory):
     subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-o", so,
                     os.path.join(os.path.dirname(__file__), "hip_recorder.c")], check=True)
 
-    def run(layer, calls, limit=None, env=()):
-        r = subprocess.run([sys.executable, "-c", DRIVER, so], input=json.dumps(dict(layer=layer, calls=calls, limit=limit)),
-                           capture_output=True, text=True, env=dict(os.environ, PYTHONPATH=PKG, **dict(env)))
+    def run(layer, calls, limit=None, env=(), shared=0):
+        r = subprocess.run([sys.executable, "-c", DRIVER, so], capture_output=True, text=True,
+                           input=json.dumps(dict(layer=layer, calls=calls, limit=limit, shared=shared)), env=dict(os.environ, PYTHONPATH=PKG, **dict(env)))
         assert r.returncode == 0, r.stderr[-2000:]
         got = json.loads(r.stdout.strip().split("\n")[-1])
         names = subprocess.run(["c++filt"], input="\n".join(g[2].replace("\n", " ") for g in got), capture_output=True,
@@ -122,13 +123,13 @@ def test_chain_pass_sizes(launches, Ks, M, slots):
         assert gemms == want, call[2]
 
 
-@pytest.mark.parametrize("layer,M,per_cu", [
-    (B, 2, (3, 5)), (B, 3, (5, 4)), (B, 4, (6, 4)), (B, 8, (4, 4)),
-    ((4096, 2048, (3, 3, 3)), 3, (6, 6)), ((4096, 2048, (3, 3, 3)), 4, (4, 4)),
+@pytest.mark.parametrize("layer,M,shared,per_cu", [
+    (B, 2, 0, (3, 5)), (B, 3, 0, (5, 4)), (B, 4, 0, (6, 4)), (B, 8, 0, (4, 4)), (B, 2, 1, (3, 5)), (B, 4, 1, (4, 4)),
+    ((4096, 2048, (3, 3, 3)), 3, 0, (6, 6)), ((4096, 2048, (3, 3, 3)), 4, 0, (4, 4)),
 ])
-def test_relay_workgroups_per_cu(launches, layer, M, per_cu):
+def test_relay_workgroups_per_cu(launches, layer, M, shared, per_cu):
     """The one-wave relay launches' LDS lets a CU (160 KB) hold the launch's share of workgroups where the registers take
-    that many (6), else 4."""
-    _, (rc, err, names) = launches((288, *layer), [(M, 8, EXACT, 0)])
+    that many (6; on a context told of other work beside it 5), else 4."""
+    _, (rc, err, names) = launches((288, *layer), [(M, 8, EXACT, 0)], shared=shared)
     assert (rc, err, names) == (0, "", ["gu_relay_kernel<3, 1>", "dn_relay_kernel<3, 1>"])
     assert tuple(163840 // lds for lds in launches.lds[1]) == per_cu
