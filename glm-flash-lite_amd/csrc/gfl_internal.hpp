@@ -146,8 +146,8 @@ int launch_chains_gate_up(const uint64_t* ptrs, const int64_t* sel, const void* 
                           uint16_t* ygu, float* xd, const float* silu_tab, float act_limit, hipStream_t st);
 int launch_chains_down(const uint64_t* ptrs, int P, int topk, int E, int H, int I, int Kg, int Ku, int Kd, const GPlan& g,
                        int cap, const float* xd, uint16_t* yraw, float* out, hipStream_t st);
-// The grouped plan alone (first three launches of launch_grouped): slots, offsets, job order per token.
-// ptrs may be NULL (tok_svh is then 0).
+// The grouped plan alone (the first launches of launch_grouped: one up to GP_PLAN_CHUNK picks, else three): slots, offsets, job
+// order per token, GEMM items of passes of mt slots. ptrs may be NULL (tok_svh is then 0).
 void launch_grouped_plan(const uint64_t* ptrs, const int64_t* sel, const void* w, int w_half, int P, int topk, int E,
                          int mt, const GPlan& g, hipStream_t st);
 

@@ -564,9 +564,10 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_act_kernel(const uint64_t* __re
 // paid once per CU. At M = 8192 it moves its 604 MB at 3.1 TB/s (before 2.2). Measured, gp_act_kernel -> this one, us, MFMA grouped
 // inputs | fp32 chain inputs, E = 288: M = 250 12.2 -> 15.6 | 12.7 -> 15.1, M = 512 19.4 -> 17.8 | 20.6 -> 18.1, M = 768
 // 27.2 -> 27.9 | 29.6 -> 27.9, M = 1024 34.7 -> 30.3 | 39.4 -> 29.9, M = 2048 71.0 -> 56.9 | 74.6 -> 51.0, M = 8192 274 ->
-// 196 | 299 -> 185: taken from 8,192 picks on, where every wave has at least two items at I = 1536.
+// 196 | 299 -> 185: taken from 8,192 picks on: from there every measured size gains (at I = 1536 a wave has two items
+// there; other I, which change a slot's items, and calls with skipped picks were not measured for the line).
 constexpr int GL_NW = 16;          // waves per workgroup
-constexpr int GL_CUS = 256;        // workgroups: one per CU
+constexpr int GL_CUS = 256;        // workgroups: one per CU of an undivided MI355X
 constexpr int GL_MIN = 8192;       // picks from which the launch is taken
 constexpr int GL_LO = 3 << 10;     // first fp16 pattern held (2^-12), and how many of each sign
 constexpr int GL_N = 16 << 10;
@@ -739,8 +740,8 @@ struct GemmArgs
     uint16_t* yout;            // [mats][cap][ndim] fp16: out_block's leading r16 (ft_core.h:109) applied here
 };
 
-// Grid: 8 * ceil(E / 8) * (ndim / 256) * matrices, XCD-major. Workgroup = 8 waves x 2 tile columns = 256 output
-// columns of one matrix of one expert; the expert's slots go through in passes of GP_MT. Per group of 8 tile rows every
+// Grid: 8 * ceil(items / 8) * (ndim / 256) * matrices, XCD-major. Workgroup = 8 waves x 2 tile columns = 256 output
+// columns of one matrix for one item, a pass of up to GP_MT slots of an expert. Per group of 8 tile rows every
 // wave decodes its 16 tiles and, per pair of tile rows, reads one A fragment (16 slots x 32 k) per row block of the
 // pass and runs 2 MFMAs (16x16x32) with it, one per column. The tiles stream through per-wave LDS rings and the slots'
 // inputs through a shared ring, both filled by LDS-direct loads GP_NG - 1 groups ahead; one workgroup barrier per group
@@ -756,8 +757,8 @@ __global__ __launch_bounds__(GP_NW * 64) void gp_gemm_kernel(GemmArgs a)
     // the wave index in a scalar register, so every LDS-DMA destination (M0) is scalar arithmetic
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     // XCD-aware order: workgroups are dispatched round-robin over the 8 XCDs (XCD = linear id % 8), so every
-    // workgroup of the ei-th expert of the dispatch order gets a linear id = ei (mod 8) and the expert's slot inputs
-    // are fetched into one L2
+    // workgroup of the it-th item of the dispatch order gets a linear id = it (mod 8) and the item's slot inputs are
+    // fetched into one L2
     const int nch = a.ndim / GP_WCOLS, per = nch * a.nmat;
     const int xcd = blockIdx.x % 8, j = blockIdx.x / 8;
     const int it = (j / per) * 8 + xcd, rr0 = j % per;
@@ -769,7 +770,7 @@ __global__ __launch_bounds__(GP_NW * 64) void gp_gemm_kernel(GemmArgs a)
     const int TN = a.ndim / 16, TK = a.kdim / 16, ngroups = TK / 8;
     const int t0 = (nc * GP_NW + wave) * GP_CPW;                     // this wave's first tile column
     uint8_t* ring = gp_lds + wave * NG * GB;                          // [NG][8 tile rows][GP_CPW columns][TB]
-    uint16_t* xring = reinterpret_cast<uint16_t*>(gp_lds + GP_NW * NG * GB);   // [NG][64 slots][GP_XS]
+    uint16_t* xring = reinterpret_cast<uint16_t*>(gp_lds + GP_NW * NG * GB);   // [NG][GP_MT slots][GP_XS]
     const uint8_t* tr = reinterpret_cast<const uint8_t*>(a.ptrs[(size_t)e * 9 + mat]);
     const size_t gstride = (size_t)TN * TB;                           // bytes per tile row of the matrix
     uint8_t* cb = const_cast<uint8_t*>(uniform_ptr(tr + (size_t)t0 * TB));
@@ -1073,8 +1074,9 @@ __global__ __launch_bounds__(GP_NW * 64) __attribute__((amdgpu_waves_per_eu(4)))
 // of fused multiply-adds in the reference's order, so the results are bit-identical to the decode path's.
 //
 // What bounds it: issue. Per tile about 80 cycles of VALU decode plus 8 cycles per slot of fp32 MFMA, which do not
-// overlap (the fp32 MFMA holds the SIMD's FMA units). At config 4 (M = 2048, 57 slots per expert) that sums to 6.4 ms
-// of the two GEMMs' 6.75 ms.
+// overlap (the fp32 MFMA holds the SIMD's FMA units). Counters of the gate|up launch, shares of the SIMDs' cycles with the
+// MFMAs busy / issuing other VALU / both: 64-slot passes (M = 2048, 57 slots per expert) 78 / 14 / 2%, 32-slot ones (M = 333,
+// 3 of 4 picks held) 48 / 40 / 6%, 16-slot ones (M = 64) 26 / 76 / 10%; 10-18% are neither.
 
 constexpr int XG_NW = 8;                    // waves per workgroup: 8 tile columns share one input ring
 constexpr int XG_MS = 64;                   // most slots per pass (xg_slots picks 16, 32 or 64 for a call)
@@ -1347,8 +1349,8 @@ static int gw_gemm_launch(const GemmArgs& a, int nmat, hipStream_t st)
     return 0;
 }
 
-// Slots per pass of an MFMA call of P picks over E experts: passes of GP_MT while an expert's mean share fits one with
-// room for its spread (measured at gw_gemm_kernel).
+// Slots per pass of an MFMA call of P picks (skipped ones included) over E experts: passes of GP_MT while an expert's mean
+// share fits one with room for its spread (measured at gw_gemm_kernel).
 static int gp_slots(int P, int E) { return P < 72 * E ? GP_MT : GW_MT; }
 
 template <int K>
@@ -1383,10 +1385,11 @@ static int xg_gemm_launch(const XgArgs& a, int nmat, hipStream_t st)
     return 0;
 }
 
-// Slots per pass of a call of P picks over E experts: 16 below 8 picks per expert, 32 below 28, else 64. A smaller pass leaves
-// more waves per SIMD, a larger one decodes an expert's weights less often. Measured at E = 288, top-8, 3 bits (ms per layer
-// with 16 / 32 / 64; P / E in brackets): M = 64 [1.8] 1.05 / 1.07 / 1.27, M = 333 [9.3] 1.62 / 1.64 / 1.80, M = 500 [14] 2.75 /
-// 2.59 / 2.77, M = 700 [19] 3.71 / 3.12 / 3.35, M = 1024 [28] 5.05 / 4.21 / 4.22, M = 2048 [57] 9.39 / 7.84 / 7.07.
+// Slots per pass of a call of P picks (skipped ones included: the host does not see them) over E experts: 16 below 8 picks per
+// expert, 32 below 28, else 64. A smaller pass leaves more waves per SIMD, a larger one decodes an expert's weights less
+// often. Measured at E = 288, top-8, 3 bits (ms per layer with 16 / 32 / 64; P / E in brackets): M = 64 [1.8] 1.05 / 1.07 / 1.27,
+// M = 333 [9.3] 1.62 / 1.64 / 1.80, M = 500 [14] 2.75 / 2.59 / 2.77, M = 700 [19] 3.71 / 3.12 / 3.35, M = 1024 [28] 5.05 / 4.21 / 4.22,
+// M = 2048 [57] 9.39 / 7.84 / 7.07.
 // With 5 bits a 64-slot pass takes 84 KB of LDS, one workgroup per CU (2 waves per SIMD): where all three matrices have 5, 32
 // slots from 28 picks on too, and where two have, below 48 picks (64 -> 32 slots, ms; bits gate/up/down): 5/5/5 M = 1024 5.55
 // -> 4.56, M = 1500 6.83 -> 6.54, M = 2048 8.68 -> 8.34, M = 4096 16.7 -> 15.6, E = 72 M = 300 [33] 1.63 -> 1.41, M = 1200 [133]
@@ -1394,6 +1397,10 @@ static int xg_gemm_launch(const XgArgs& a, int nmat, hipStream_t st)
 // -> 8.13 and 8.13 -> 8.22, M = 4096 [114] 15.8 -> 15.5; 5/2/5 M = 1024 5.26 -> 4.41, M = 1500 6.56 -> 6.43, M = 2048 8.24 ->
 // 8.17 and 8.21 -> 8.21. With one matrix of 5 bits 64 stays: 3/3/5 M = 1500 5.99 -> 6.33, M = 2048 7.72 -> 8.08, M = 4096 15.1
 // -> 15.4 (but M = 1024 4.72 -> 4.37); 3/5/4 M = 2048 7.74 -> 8.13.
+// A rank that holds 72 of 288 experts and skips the other picks (us with 16 / 32 / 64): M = 64 [7.1] 316 / 318 / 363, M = 128
+// [14] 412 / 421 / 467, M = 333 [37] 612 / 616 / 651, M = 1024 [114] 1368 / 1162 / 1148, M = 2048 [228] 2506 / 2109 / 1900; all 288
+// registered and 3 of 4 picks skipped: M = 128 [3.6] 733 / 767 / 895, M = 333 1269 / 1281 / 1415, M = 1024 [28] 1982 / 1972 / 2102,
+// M = 2048 [57] 2927 / 2673 / 2823: the size chosen is up to 7% from the best of the three.
 static int xg_slots(int P, int E, int Kg, int Ku, int Kd)
 {
     const int five = (Kg == 5) + (Ku == 5) + (Kd == 5);

@@ -113,11 +113,12 @@ int gfl_layer_info(gfl_ctx* ctx, int li, int* info);
  * buffer may be NULL); topk = 0 writes M rows of zeros to out (sel and w may be NULL).
  * M*topk <= 64, and up to 1024 with fewer than half a pick per expert of the layer (three quarters where gate and up
  * have different bits), mode MFMA or an out that is not 16-byte aligned: the decode launches. Other calls up to
- * M*topk = 65536 (EXACT modes only; MFMA is refused above 1024): the grouped plan of the prefill path, then the reference's accumulator chains (each chain step one element of a K=1
- * fp32 MFMA, i.e. an fmaf), each weight decoded once per pass of up to 64 of an expert's slots, bit-identical to the
- * reference's EXACT mode at any batch size. Above 1024 picks out must be 16-byte aligned too and M*topk*max(H, I) <
- * 2^29. That path uses the prefill workspace: gfl_register_layer reserves it for 1024 picks, gfl_grouped_reserve sizes it
- * for more ahead of graph capture (otherwise the first call of a larger size grows it). */
+ * M*topk = 65536 (EXACT modes only; MFMA is refused above 1024): the grouped plan of the prefill path, then the
+ * reference's accumulator chains (each chain step one element of a K=1 fp32 MFMA, i.e. an fmaf), each weight decoded
+ * once per pass of up to 64 of an expert's slots, bit-identical to the reference's EXACT mode at any batch size. Above
+ * 1024 picks out must be 16-byte aligned too and M*topk*max(H, I) < 2^29. That path uses the prefill workspace:
+ * gfl_register_layer reserves it for 1024 picks, gfl_grouped_reserve sizes it for more ahead of graph capture
+ * (otherwise the first call of a larger size grows it). */
 int gfl_moe_forward(gfl_ctx* ctx, int li, const uint16_t* x, const int64_t* sel, const void* w, int w_is_half, int M,
                     int topk, float* out, int mode, float act_limit, gfl_stream stream);
 
@@ -155,8 +156,8 @@ int gfl_moe_forward_shared(gfl_ctx* ctx, int li, const uint16_t* x, const int64_
 int gfl_moe_forward_noalloc(gfl_ctx* ctx, int li, const uint16_t* x, const int64_t* sel, const void* w,
                             int w_is_half, int M, int topk, float* out, int mode, float act_limit, gfl_stream stream);
 
-/* mode: AUTO, AFFINE, EXACT or I16 (all computed bit-exact to EXACT), or MFMA. With MFMA the workgroups of a routed expert take up to 4 of its slots
- * per pass, so the expert's tiles are decoded once for all of them.
+/* mode: AUTO, AFFINE, EXACT or I16 (all computed bit-exact to EXACT), or MFMA. With MFMA the workgroups of a routed expert
+ * take up to 4 of its slots per pass, so the expert's tiles are decoded once for all of them.
  * Environment: GFL_SLOTS_PER_PASS = 1, 2, 4 or 8 forces the number of (token, expert) slots one GEMV pass of the decode
  * launches accumulates (default: 1 up to M = 8, with a workgroup per slot; else 2, with a workgroup per expert
  * whose slots take passes; MFMA: min(M, 4)), and keeps calls of up to 1024 picks on them. Read once by gfl_ctx_create. */
@@ -273,7 +274,7 @@ int gfl_stats(gfl_ctx* ctx, int64_t* out, int n);
 /* Per-stage device timing of gfl_moe_forward, the counterpart of the per-phase wall times tier_stats reports
  * (ft_tier_ext.cpp:906-914): while enabled, every forward brackets its launches with device events. Stage 1 is the
  * gate|up launch (routing plan, gate|up GEMV, SwiGLU and down-input prep), stage 3 the down launch (down GEMV,
- * output transform, weighted combine); stage 2 is a whole gfl_grouped_forward call (its eight launches); stages 0 and
+ * output transform, weighted combine); stage 2 is a whole gfl_grouped_forward call; stages 0 and
  * 4 (plan, combine) run inside the other launches and stay 0.
  * gfl_profile_read synchronises the recorded events, adds their elapsed milliseconds into stage_ms[5] and launch
  * counts into launches[5] (host arrays), and clears the record. */
