@@ -680,12 +680,12 @@ static int run_chains(gfl_ctx* c, const Layer& L, const uint16_t* x, const int64
 //   H = 2048, I = 768: M = 9 75 -> 82, M = 16 117 -> 117, M = 24 153 -> 142; gate 3 and up 5 bits M = 22 157 -> 165,
 //     M = 27 181 -> 177
 //   E = 72: M = 9 [1] 259 -> 240, M = 64 [7.1] 1250 -> 526
-// The host does not see skipped picks. Of 288 experts' picks with only 72 held (E = 72 registered): M = 9 133 -> 112, M = 18
-// 232 -> 156, M = 64 550 -> 303, M = 128 979 -> 399; 36 held: M = 9 157 -> 93; all registered, 3 of 4 picks skipped: M = 18 238
-// -> 178, M = 64 672 -> 480; 19 of 20 skipped: M = 18 156 -> 82; all: M = 18 105 -> 24.
-// Up to 64 picks the relay launches stay, which are faster from about 36 experts on (relay -> chains): E = 72 M = 5 165 -> 189,
-// M = 8 248 -> 267, E = 128 M = 8 250 -> 265 (Zipf 246 -> 239), H = 2048 E = 72 M = 8 62 -> 84, E = 36 M = 5 166 -> 188; not with many
-// picks on few: E = 36 M = 8 246 -> 207, E = 8 M = 5 154 -> 116, M = 8 224 -> 122.
+// The host does not see skipped picks. Of 288 experts' picks with only 72 held (E = 72 registered): M = 9 133 -> 112, M
+// = 18 232 -> 156, M = 64 550 -> 303, M = 128 979 -> 399; 36 held: M = 9 157 -> 93; all registered, 3 of 4 picks
+// skipped: M = 18 238 -> 178, M = 64 672 -> 480; 19 of 20 skipped: M = 18 156 -> 82; all: M = 18 105 -> 24.
+// Up to 64 picks the relay launches stay, which are faster from about 36 experts on (relay -> chains): E = 72 M = 5 165
+// -> 189, M = 8 248 -> 267, E = 128 M = 8 250 -> 265 (Zipf 246 -> 239), H = 2048 E = 72 M = 8 62 -> 84, E = 36 M = 5
+// 166 -> 188; not with many picks on few: E = 36 M = 8 246 -> 207, E = 8 M = 5 154 -> 116, M = 8 224 -> 122.
 // The chains' combine writes 16 bytes at a time, and the forced launch shapes (GFL_SLOTS_PER_PASS, GFL_RELAY) name the
 // decode launches, so an unaligned out and a context with either keep those; so does one whose registration found no memory
 // for the chains' workspace.

@@ -557,15 +557,16 @@ __global__ __launch_bounds__(GP_TW * 64) void gp_act_kernel(const uint64_t* __re
     }
 }
 
-// The same for calls of many picks, with the middle of the silu table in LDS. Each gate element is a lookup at an address
-// of its own, which from L1 takes the kernel a cycle per lane: at M = 8192 (top-8, I = 1536) about 160 of its 274 us. A
-// workgroup of 16 waves fills a CU's registers, holds the binades [2^-12, 16) of both signs (128 KB; other gates read
-// the table in memory) and goes through the (slot, 12 blocks) items, consecutive ones side by side, so that the fill is
-// paid once per CU. At M = 8192 it moves its 604 MB at 3.1 TB/s (before 2.2). Measured, gp_act_kernel -> this one, us, MFMA grouped
-// inputs | fp32 chain inputs, E = 288: M = 250 12.2 -> 15.6 | 12.7 -> 15.1, M = 512 19.4 -> 17.8 | 20.6 -> 18.1, M = 768
-// 27.2 -> 27.9 | 29.6 -> 27.9, M = 1024 34.7 -> 30.3 | 39.4 -> 29.9, M = 2048 71.0 -> 56.9 | 74.6 -> 51.0, M = 8192 274 ->
-// 196 | 299 -> 185: taken from 8,192 picks on: from there every measured size gains (at I = 1536 a wave has two items
-// there; other I, which change a slot's items, and calls with skipped picks were not measured for the line).
+// The same for calls of many picks, with the middle of the silu table in LDS. Each gate element is a lookup at an
+// address of its own, which from L1 takes the kernel a cycle per lane: at M = 8192 (top-8, I = 1536) about 160 of its
+// 274 us. A workgroup of 16 waves fills a CU's registers, holds the binades [2^-12, 16) of both signs (128 KB; other
+// gates read the table in memory) and goes through the (slot, 12 blocks) items, consecutive ones side by side, so that
+// the fill is paid once per CU. At M = 8192 it moves its 604 MB at 3.1 TB/s (before 2.2). Measured, gp_act_kernel ->
+// this one, us, MFMA grouped inputs | fp32 chain inputs, E = 288: M = 250 12.2 -> 15.6 | 12.7 -> 15.1, M = 512 19.4 ->
+// 17.8 | 20.6 -> 18.1, M = 768 27.2 -> 27.9 | 29.6 -> 27.9, M = 1024 34.7 -> 30.3 | 39.4 -> 29.9, M = 2048 71.0 -> 56.9
+// | 74.6 -> 51.0, M = 8192 274 -> 196 | 299 -> 185: taken from 8,192 picks on: from there every measured size gains (at
+// I = 1536 a wave has two items there; other I, which change a slot's items, and calls with skipped picks were not
+// measured for the line).
 constexpr int GL_NW = 16;          // waves per workgroup
 constexpr int GL_CUS = 256;        // workgroups: one per CU of an undivided MI355X
 constexpr int GL_MIN = 8192;       // picks from which the launch is taken
@@ -724,10 +725,11 @@ __device__ __forceinline__ void gp_wait_vmcnt()
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// Workgroup barrier without __syncthreads' release fence: that fence waits for vmcnt(0), i.e. for every LDS-direct
-// load still in flight, which would drain the prefetch ring at every group. Each wave has already waited for its own
-// loads of the group it is about to read; the barrier only has to order those waits and the previous group's LDS
-// reads (waited for here, nothing else is outstanding on that counter) across the waves. The "memory" clobber keeps the compiler from moving LDS accesses across it.
+// Workgroup barrier without __syncthreads' release fence: that fence waits for vmcnt(0), i.e. for every LDS-direct load
+// still in flight, which would drain the prefetch ring at every group. Each wave has already waited for its own loads
+// of the group it is about to read; the barrier only has to order those waits and the previous group's LDS reads
+// (waited for here, nothing else is outstanding on that counter) across the waves. The "memory" clobber keeps the
+// compiler from moving LDS accesses across it.
 __device__ __forceinline__ void gp_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 struct GemmArgs
@@ -898,9 +900,10 @@ __global__ __launch_bounds__(GP_NW * 64) void gp_gemm_kernel(GemmArgs a)
 // part. The accumulators take 80 VGPRs; the kernel fits 128 (4 waves per SIMD, two workgroups per CU) with groups of 4 tile
 // rows, whose input ring is 40 KB, and one input fragment in flight at a time. The input rows are swizzled instead of
 // padded: a load brings two rows, and their 128-byte chunks have to lie next to each other in LDS.
-// Measured against passes of 80 (ms per layer, E = 288 top-8, mean slots in brackets): M = 2048 [57] 1.60 -> 1.70, M = 2500
-// [69] 1.76 -> 1.80, M = 2700 [75] 2.00 -> 1.87, M = 4096 [114] 3.07 -> 2.42, M = 5000 [139] 3.43 -> 2.80, M = 8192 [228] 5.42 -> 4.86. Passes of 144:
-// 4096 2.41, 5000 3.02, 8192 4.80; of 176 (two registers spilled): 2.43, 2.80, 4.99.
+// Measured against passes of 80 (ms per layer, E = 288 top-8, mean slots in brackets): M = 2048 [57] 1.60 -> 1.70, M =
+// 2500 [69] 1.76 -> 1.80, M = 2700 [75] 2.00 -> 1.87, M = 4096 [114] 3.07 -> 2.42, M = 5000 [139] 3.43 -> 2.80, M =
+// 8192 [228] 5.42 -> 4.86. Passes of 144: 4096 2.41, 5000 3.02, 8192 4.80; of 176 (two registers spilled): 2.43, 2.80,
+// 4.99.
 constexpr int GW_MT = 160;         // slots per pass (up to 10 MFMA row blocks)
 constexpr int GW_GR = 4;           // tile rows per group
 constexpr int GW_XPW = GW_MT / 2 / GP_NW;       // pairs of input rows each wave loads per group
@@ -1076,7 +1079,7 @@ __global__ __launch_bounds__(GP_NW * 64) __attribute__((amdgpu_waves_per_eu(4)))
 // What bounds it: issue. Per tile about 80 cycles of VALU decode plus 8 cycles per slot of fp32 MFMA, which do not
 // overlap (the fp32 MFMA holds the SIMD's FMA units). Counters of the gate|up launch, shares of the SIMDs' cycles with the
 // MFMAs busy / issuing other VALU / both: 64-slot passes (M = 2048, 57 slots per expert) 78 / 14 / 2%, 32-slot ones (M = 333,
-// 3 of 4 picks held) 48 / 40 / 6%, 16-slot ones (M = 64) 26 / 76 / 10%; 10-18% are neither.
+// 3 of 4 picks held) 48 / 40 / 6%, 16-slot ones (M = 64) 26 / 76 / 10%; 8-18% are neither.
 
 constexpr int XG_NW = 8;                    // waves per workgroup: 8 tile columns share one input ring
 constexpr int XG_MS = 64;                   // most slots per pass (xg_slots picks 16, 32 or 64 for a call)
@@ -1385,22 +1388,23 @@ static int xg_gemm_launch(const XgArgs& a, int nmat, hipStream_t st)
     return 0;
 }
 
-// Slots per pass of a call of P picks (skipped ones included: the host does not see them) over E experts: 16 below 8 picks per
-// expert, 32 below 28, else 64. A smaller pass leaves more waves per SIMD, a larger one decodes an expert's weights less
-// often. Measured at E = 288, top-8, 3 bits (ms per layer with 16 / 32 / 64; P / E in brackets): M = 64 [1.8] 1.05 / 1.07 / 1.27,
-// M = 333 [9.3] 1.62 / 1.64 / 1.80, M = 500 [14] 2.75 / 2.59 / 2.77, M = 700 [19] 3.71 / 3.12 / 3.35, M = 1024 [28] 5.05 / 4.21 / 4.22,
-// M = 2048 [57] 9.39 / 7.84 / 7.07.
-// With 5 bits a 64-slot pass takes 84 KB of LDS, one workgroup per CU (2 waves per SIMD): where all three matrices have 5, 32
-// slots from 28 picks on too, and where two have, below 48 picks (64 -> 32 slots, ms; bits gate/up/down): 5/5/5 M = 1024 5.55
-// -> 4.56, M = 1500 6.83 -> 6.54, M = 2048 8.68 -> 8.34, M = 4096 16.7 -> 15.6, E = 72 M = 300 [33] 1.63 -> 1.41, M = 1200 [133]
-// 5.07 -> 4.62, H = 4096 I = 2048 M = 2048 9.26 -> 8.78; 5/5/3 M = 1024 5.14 -> 4.40, M = 1500 [42] 6.45 -> 6.40, M = 2048 8.13
-// -> 8.13 and 8.13 -> 8.22, M = 4096 [114] 15.8 -> 15.5; 5/2/5 M = 1024 5.26 -> 4.41, M = 1500 6.56 -> 6.43, M = 2048 8.24 ->
-// 8.17 and 8.21 -> 8.21. With one matrix of 5 bits 64 stays: 3/3/5 M = 1500 5.99 -> 6.33, M = 2048 7.72 -> 8.08, M = 4096 15.1
-// -> 15.4 (but M = 1024 4.72 -> 4.37); 3/5/4 M = 2048 7.74 -> 8.13.
-// A rank that holds 72 of 288 experts and skips the other picks (us with 16 / 32 / 64): M = 64 [7.1] 316 / 318 / 363, M = 128
-// [14] 412 / 421 / 467, M = 333 [37] 612 / 616 / 651, M = 1024 [114] 1368 / 1162 / 1148, M = 2048 [228] 2506 / 2109 / 1900; all 288
-// registered and 3 of 4 picks skipped: M = 128 [3.6] 733 / 767 / 895, M = 333 1269 / 1281 / 1415, M = 1024 [28] 1982 / 1972 / 2102,
-// M = 2048 [57] 2927 / 2673 / 2823: the size chosen is up to 7% from the best of the three.
+// Slots per pass of a call of P picks (skipped ones included: the host does not see them) over E experts: 16 below 8
+// picks per expert, 32 below 28, else 64. A smaller pass leaves more waves per SIMD, a larger one decodes an expert's
+// weights less often. Measured at E = 288, top-8, 3 bits (ms per layer with 16 / 32 / 64; P / E in brackets): M = 64
+// [1.8] 1.05 / 1.07 / 1.27, M = 333 [9.3] 1.62 / 1.64 / 1.80, M = 500 [14] 2.75 / 2.59 / 2.77, M = 700 [19] 3.71 / 3.12
+// / 3.35, M = 1024 [28] 5.05 / 4.21 / 4.22, M = 2048 [57] 9.39 / 7.84 / 7.07.
+// With 5 bits a 64-slot pass takes 84 KB of LDS, one workgroup per CU (2 waves per SIMD): where all three matrices have
+// 5, 32 slots from 28 picks on too, and where two have, below 48 picks (64 -> 32 slots, ms; bits gate/up/down): 5/5/5 M
+// = 1024 5.55 -> 4.56, M = 1500 6.83 -> 6.54, M = 2048 8.68 -> 8.34, M = 4096 16.7 -> 15.6, E = 72 M = 300 [33] 1.63 ->
+// 1.41, M = 1200 [133] 5.07 -> 4.62, H = 4096 I = 2048 M = 2048 9.26 -> 8.78; 5/5/3 M = 1024 5.14 -> 4.40, M = 1500
+// [42] 6.45 -> 6.40, M = 2048 8.13 -> 8.13 and 8.13 -> 8.22, M = 4096 [114] 15.8 -> 15.5; 5/2/5 M = 1024 5.26 -> 4.41,
+// M = 1500 6.56 -> 6.43, M = 2048 8.24 -> 8.17 and 8.21 -> 8.21. With one matrix of 5 bits 64 stays: 3/3/5 M = 1500
+// 5.99 -> 6.33, M = 2048 7.72 -> 8.08, M = 4096 15.1 -> 15.4 (but M = 1024 4.72 -> 4.37); 3/5/4 M = 2048 7.74 -> 8.13.
+// A rank that holds 72 of 288 experts and skips the other picks (us with 16 / 32 / 64): M = 64 [7.1] 316 / 318 / 363, M
+// = 128 [14] 412 / 421 / 467, M = 333 [37] 612 / 616 / 651, M = 1024 [114] 1368 / 1162 / 1148, M = 2048 [228] 2506 /
+// 2109 / 1900; all 288 registered and 3 of 4 picks skipped: M = 128 [3.6] 733 / 767 / 895, M = 333 1269 / 1281 / 1415,
+// M = 1024 [28] 1982 / 1972 / 2102, M = 2048 [57] 2927 / 2673 / 2823: the size chosen is up to 7% from the best of the
+// three.
 static int xg_slots(int P, int E, int Kg, int Ku, int Kd)
 {
     const int five = (Kg == 5) + (Ku == 5) + (Kd == 5);
