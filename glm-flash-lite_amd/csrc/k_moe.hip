@@ -1852,7 +1852,10 @@ static void gu_relay_launch(const GuArgs& a, int nmat, int beside, hipStream_t s
     const size_t lds = balanced_lds(gu_relay_lds<K>(a.H, a.P, a.E), held);
     GuArgs b = a;
     b.nmat_launch = nmat;
-    b.prio = relay_prio(a.prio, nwg * GU_NW, held);
+    // with 6 waves per SIMD a short column's waves end together without it (us per 4 layers off -> on: M = 8 I = 768 at H =
+    // 2048 230 -> 233, H = 3072 324 -> 317, H = 4096 412 -> 403, H = 5120 510 -> 496; M = 4 I = 1536 at H = 2048 221 -> 224; 5 waves
+    // per SIMD, M = 6 I = 768 at H = 2048, 8 layers, 378 -> 359)
+    b.prio = a.prio < 0 && held > 5 && a.H < 24 * 128 ? 0 : relay_prio(a.prio, nwg * GU_NW, held);
     timed_launch(kern, dim3(8 + relay_blocks(nwg, RW)), dim3(GU_NW * 64), lds, st, b);
 }
 
